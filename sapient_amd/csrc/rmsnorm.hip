@@ -21,13 +21,16 @@
 //    streaming them past the caches measured ~+20 % achieved bandwidth on
 //    MI355X. The weight row uses ordinary loads (it is re-read by every row).
 //  - The residual store is issued before the reduction, overlapping it.
-//  - Rows wider than 16 waves x 16 values, or whose pointers / width do not
-//    allow 16-byte access, take a block-per-row two-pass kernel.
+//  - Rows whose pointers or width do not allow aligned 16-byte access are held in
+//    registers too, in runs at element alignment (rms_rows_ragged); rows wider
+//    than 16 waves hold take a block-per-row two-pass kernel.
 //
 // Parity: x·x, the division by dim, sqrt and 1/· are IEEE-rounded f32 exactly
 // as in the reference; the products y = (r·inv)·w round in the same order (the
 // file is compiled with -ffp-contract=off). Only the order of the Σ differs
 // (per-lane serial, then a tree), which moves ms by a few f32 ulps.
+#include <type_traits>
+
 #include "sph_common.h"
 
 namespace sph {
@@ -238,6 +241,108 @@ __global__ __launch_bounds__(W >= 4 ? 64 * W : 256) void rms_rows_vec(const TX* 
     }
 }
 
+// Rows whose width no 16-byte vector divides, or whose pointers are only element-aligned: the row
+// is split and held in registers as in rms_rows_vec (one read of every input), each lane moving
+// 16-byte runs at whatever alignment its row has; the lane whose run crosses the row's end moves
+// its last elements one by one. HBM-bound; the straddled cache lines cost about a third over the
+// aligned kernel. Against rms_rows_generic (three passes of element accesses) on MI355X: add +
+// RMSNorm f16 4099 x 2565 29.1 -> 20.7 µs, f32 53.4 -> 31.2, bf16 16384 x 4095 222 -> 145; RMSNorm
+// bf16 16384 x 4095 143 -> 74; LayerNorm 176 -> 80. Shifting every lane's runs to 16- or 128-byte
+// boundaries of the row (all full runs aligned) was slower in every case (RMSNorm 74 -> 82-83):
+// both ends of a row then move element by element.
+// weight and bias are f32 (wb_f32) or TX.
+template <typename TX, typename TO, int KIND, int W, int VPT, bool NT>
+__global__ __launch_bounds__(W >= 4 ? 64 * W : 256) void rms_rows_ragged(const TX* __restrict__ x, TX* __restrict__ residual,
+                                                                     TX* __restrict__ sum, const void* __restrict__ w,
+                                                                     const void* __restrict__ bias, bool wb_f32,
+                                                                     TO* __restrict__ out, int64_t rows, int dim,
+                                                                     float eps) {
+    constexpr int E = vec16<TX>::n;
+    constexpr int WPB = W >= 4 ? W : 4;
+    constexpr int RPB = WPB / W;
+    __shared__ float partial[2][WPB];
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wv = threadIdx.x / kWave;
+    const int64_t row = (int64_t)blockIdx.x * RPB + wv / W;
+    const bool live = row < rows;  // rows past the end still meet the block's barriers
+    const size_t base = (size_t)(live ? row : 0) * (size_t)dim;
+    const int e0 = ((wv % W) * VPT * kWave + lane) * E;  // this lane's first element; its runs lie kWave * E apart
+
+    u32x4 cx[VPT], cres[VPT];
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) {
+        const int i = e0 + j * kWave * E;
+        if (live && i < dim) {
+            cx[j] = load_run16<TX, NT>(x + base + i, dim - i);
+            if constexpr (adds(KIND)) cres[j] = load_run16<TX, NT>(residual + base + i, dim - i);
+        }
+    }
+    float r[VPT][E];
+    float ss = 0.0f;
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) {
+        const int i = e0 + j * kWave * E;
+        if (live && i < dim) {
+            unpack16<TX, E>(cx[j], r[j]);  // elements past the row's end are 0 and add nothing
+            if constexpr (adds(KIND)) {
+                float b[E];
+                unpack16<TX, E>(cres[j], b);
+#pragma unroll
+                for (int e = 0; e < E; ++e) r[j][e] = r[j][e] + b[e];
+                store_run_f32<TX, E, NT>((KIND == K_ADD_RMS_TO ? sum : residual) + base + i, dim - i, r[j]);
+            }
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                if constexpr (KIND == K_LAYER) ss = ss + r[j][e];
+                else ss = ss + r[j][e] * r[j][e];
+            }
+        }
+    }
+    ss = row_sum<W, WPB>(ss, partial, 0, lane, wv);
+    float inv;
+    if constexpr (KIND == K_LAYER) {
+        const float mean = ss / (float)dim;
+        float vs = 0.0f;
+#pragma unroll
+        for (int j = 0; j < VPT; ++j) {
+            const int i = e0 + j * kWave * E;
+            if (live && i < dim) {
+#pragma unroll
+                for (int e = 0; e < E; ++e) {
+                    r[j][e] = i + e < dim ? r[j][e] - mean : 0.0f;
+                    vs = vs + r[j][e] * r[j][e];
+                }
+            }
+        }
+        vs = row_sum<W, WPB>(vs, partial, 1, lane, wv);
+        inv = 1.0f / sqrtf(vs / (float)dim + eps);
+    } else {
+        inv = 1.0f / sqrtf(ss / (float)dim + eps);
+    }
+    auto load_wb = [&](const void* p, int i, float absent, float (&v)[E]) {
+        if (p == nullptr) {
+#pragma unroll
+            for (int e = 0; e < E; ++e) v[e] = absent;
+        } else if (wb_f32) {
+            load_run_f32<float, E, false>(static_cast<const float*>(p) + i, dim - i, v);
+        } else {
+            load_run_f32<TX, E, false>(static_cast<const TX*>(p) + i, dim - i, v);
+        }
+    };
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) {
+        const int i = e0 + j * kWave * E;
+        if (live && i < dim) {
+            float wj[E], bj[E], y[E];
+            load_wb(w, i, 1.0f, wj);
+            load_wb(KIND == K_LAYER ? bias : nullptr, i, -0.0f, bj);
+#pragma unroll
+            for (int e = 0; e < E; ++e) y[e] = norm_out<KIND>(r[j][e], inv, wj[e], bj[e]);
+            store_run_f32<TO, E, NT>(out + base + i, dim - i, y);
+        }
+    }
+}
+
 // Any width and alignment: one 256-thread block per row, re-reading the row
 // from cache for each pass. The last pass recomputes r from the inputs so the
 // half variants normalise the unrounded f32 sum; each thread owns the same
@@ -329,6 +434,50 @@ int launch_shape(const TX* xp, TX* rp, TX* sp, const TW* wp, const TW* bp, TO* o
                                                    stream);
 }
 
+// One launch of the ragged kernel, W waves per row (the fewest that cover it); kNoShape past 16 waves.
+template <typename TX, typename TO, int KIND, int VPT, bool NT>
+int launch_ragged(const TX* xp, TX* rp, TX* sp, const void* wp, const void* bp, bool wb_f32, TO* op, int64_t nr,
+                  int64_t dim, float eps, hipStream_t stream) {
+    constexpr int64_t kRun = (int64_t)kWave * VPT * vec16<TX>::n;  // elements of a row per wave
+    if (dim > 16 * kRun) return kNoShape;
+    int W = 1;
+    while (dim > kRun * W) W *= 2;
+    const int rpb = W >= 4 ? 1 : 4 / W;
+    const int threads = W >= 4 ? kWave * W : 256;
+    const dim3 grid((unsigned)((nr + rpb - 1) / rpb));
+    auto go = [&](auto w) {
+        return launch(rms_rows_ragged<TX, TO, KIND, decltype(w)::value, VPT, NT>, grid, threads, stream, xp, rp, sp, wp,
+                      bp, wb_f32, op, nr, (int)dim, eps);
+    };
+    switch (W) {
+    case 1: return go(std::integral_constant<int, 1>{});
+    case 2: return go(std::integral_constant<int, 2>{});
+    case 4: return go(std::integral_constant<int, 4>{});
+    case 8: return go(std::integral_constant<int, 8>{});
+    default: return go(std::integral_constant<int, 16>{});
+    }
+}
+
+// Runs per lane of a ragged launch: one where the launch is small (up to kFewValues; f16 300 x 1001
+// 4.1 µs against 4.8 with two) or fuses an f32 add (4096 x 4096 at an odd offset 45.8 against 50.5),
+// else two (RMSNorm bf16 16384 x 4095 74 against 88, LayerNorm 80 against 97). Cached accesses
+// up to kCachedBytes: f16 add 4099 x 2565 (84 MB) 20.7 against 24.2 non-temporal, at 134 MB both
+// alike, bf16 16384 x 4095 (537 MB) 152 against 145.
+template <typename TX, typename TO, int KIND>
+int launch_ragged_any(const TX* xp, TX* rp, TX* sp, const void* wp, const void* bp, bool wb_f32, TO* op, int64_t nr,
+                      int64_t dim, float eps, bool few, hipStream_t stream) {
+    const int64_t bytes = nr * dim * (int64_t)(sizeof(TX) * (adds(KIND) ? 3 : 1) + sizeof(TO));
+    const bool nt = bytes >= kCachedBytes;
+    int st = kNoShape;
+    if (few || (adds(KIND) && sizeof(TX) == 4)) {
+        st = nt ? launch_ragged<TX, TO, KIND, 1, true>(xp, rp, sp, wp, bp, wb_f32, op, nr, dim, eps, stream)
+                : launch_ragged<TX, TO, KIND, 1, false>(xp, rp, sp, wp, bp, wb_f32, op, nr, dim, eps, stream);
+    }
+    if (st != kNoShape) return st;
+    return nt ? launch_ragged<TX, TO, KIND, 2, true>(xp, rp, sp, wp, bp, wb_f32, op, nr, dim, eps, stream)
+              : launch_ragged<TX, TO, KIND, 2, false>(xp, rp, sp, wp, bp, wb_f32, op, nr, dim, eps, stream);
+}
+
 // Launch shapes, measured at 16384 x 4096 on MI355X (round-robin medians on
 // two machines; one-block-per-row shapes listed as VPT):
 //  - fused add + RMSNorm: row-looping blocks, one vector per lane, 16 (f32)
@@ -344,8 +493,8 @@ int launch_shape(const TX* xp, TX* rp, TX* sp, const TW* wp, const TW* bp, TO* o
 //    f16 47.4 µs (16 waves per CU with two vectors: 88.8, 48.9; one block per
 //    row: 92.0, 55.6).
 // A row too wide for the looping shape takes the one-block-per-row kernel
-// (twice the values per lane past 16 waves); unaligned rows, or rows wider
-// than that, the generic kernel.
+// (twice the values per lane past 16 waves); rows without aligned 16-byte access
+// the ragged kernel, and rows wider than that the generic kernel.
 constexpr int64_t kFewValues = int64_t(1) << 21;
 
 template <typename TX, typename TW, typename TO, int KIND>
@@ -400,8 +549,11 @@ int launch_rms(const void* x, void* residual, void* sum, const void* w, const vo
                 st = launch_shape<TX, TW, TO, KIND, 2 * VPT, false>(xp, rp, sp, wp, bp, op, nr, (int)dim, eps, 16, stream);
             if (st == kNoShape) return SPH_EINVAL;  // unreachable: vec_ok bounds the width
         } else {
-            st = launch(rms_rows_generic<TX, TW, TO, KIND>, dim3((unsigned)nr), 256, stream, xp, rp, sp, wp, bp, op,
-                        nr, dim, eps);
+            st = launch_ragged_any<TX, TO, KIND>(xp, rp, sp, w, bias, std::is_same<TW, float>::value, op, nr, dim, eps,
+                                                 nr * dim <= kFewValues, stream);
+            if (st == kNoShape)  // wider than 16 waves at two runs per lane
+                st = launch(rms_rows_generic<TX, TW, TO, KIND>, dim3((unsigned)nr), 256, stream, xp, rp, sp, wp, bp, op,
+                            nr, dim, eps);
         }
         if (st != SPH_OK) return st;
     }

@@ -167,6 +167,74 @@ __device__ __forceinline__ void store_f32(T* __restrict__ p, const float (&v)[N]
     store_words<T, N, NT>(p, raw);
 }
 
+// ───────────────────── runs at element alignment ─────────────────────
+// gfx950 serves 16-byte global accesses at any address (unaligned access mode, which the HSA
+// ABI always enables), so rows whose width or base no vector divides still move 16 bytes per
+// lane; only the cache lines that a wave's 1 KiB straddles are requested twice.
+typedef u32x4 u32x4_at4 __attribute__((aligned(4)));
+typedef u32x4 u32x4_at2 __attribute__((aligned(2)));
+template <typename T> struct elem_vec16 { typedef u32x4_at2 type; };
+template <> struct elem_vec16<float> { typedef u32x4_at4 type; };
+
+// The first min(n, E) of E consecutive elements (16 bytes of T) as raw words; the rest read as zero bits.
+template <typename T, bool NT>
+__device__ __forceinline__ u32x4 load_run16(const T* p, int n) {
+    constexpr int E = vec16<T>::n;
+    if (n >= E) {
+        // Not vload / vstore: a template parameter deduced from the pointer would drop its alignment.
+        const auto* a = reinterpret_cast<const typename elem_vec16<T>::type*>(p);
+        if constexpr (NT) return __builtin_nontemporal_load(a);
+        else return *a;
+    }
+    u32x4 q = {0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+        if (e < n) {
+            if constexpr (sizeof(T) == 4) q[e] = __builtin_bit_cast(uint32_t, p[e]);
+            else q[e / 2] |= (uint32_t)__builtin_bit_cast(uint16_t, p[e]) << (16 * (e & 1));
+        }
+    }
+    return q;
+}
+
+// The first min(n, N) of N consecutive elements as f32 (N a multiple of T's 16-byte run).
+template <typename T, int N, bool NT>
+__device__ __forceinline__ void load_run_f32(const T* p, int n, float (&v)[N]) {
+    constexpr int E = vec16<T>::n;
+    uint32_t raw[words_of<T, N>::n];
+#pragma unroll
+    for (int c = 0; c < N / E; ++c) {
+        const u32x4 q = load_run16<T, NT>(p + c * E, n - c * E);
+        raw[4 * c] = q.x; raw[4 * c + 1] = q.y; raw[4 * c + 2] = q.z; raw[4 * c + 3] = q.w;
+    }
+    words_to_f32<T, N>(raw, v);
+}
+
+// Store the first min(n, N) of N f32 values as consecutive elements of T.
+template <typename T, int N, bool NT>
+__device__ __forceinline__ void store_run_f32(T* p, int n, const float (&v)[N]) {
+    constexpr int E = vec16<T>::n;
+    uint32_t raw[words_of<T, N>::n];
+    f32_to_words<T, N>(v, raw);
+#pragma unroll
+    for (int c = 0; c < N / E; ++c) {
+        if (n >= (c + 1) * E) {
+            const u32x4 q = {raw[4 * c], raw[4 * c + 1], raw[4 * c + 2], raw[4 * c + 3]};
+            auto* a = reinterpret_cast<typename elem_vec16<T>::type*>(p + c * E);
+            if constexpr (NT) __builtin_nontemporal_store(q, a);
+            else *a = q;
+        } else {
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                if (c * E + e < n) {
+                    if constexpr (sizeof(T) == 4) p[c * E + e] = __builtin_bit_cast(T, raw[4 * c + e]);
+                    else p[c * E + e] = __builtin_bit_cast(T, (uint16_t)(raw[4 * c + e / 2] >> (16 * (e & 1))));
+                }
+            }
+        }
+    }
+}
+
 template <int CTRL>
 __device__ __forceinline__ float dpp_mov(float v) {
     return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));
@@ -193,6 +261,11 @@ __device__ __forceinline__ float wave_sum(float v) {
 // ─────────────────────────────── host side ───────────────────────────────
 // Compute units of the current device (cached per device); 0 if unknown.
 __attribute__((visibility("hidden"))) int device_cu_count();
+
+// Launches that move fewer bytes than this (half of the 256 MB Infinity Cache) use ordinary loads and
+// stores: their operands are mostly still in cache from the kernel before, and their results for the
+// kernel after. Non-temporal accesses, which pass the caches by, pay from there on.
+constexpr int64_t kCachedBytes = int64_t(1) << 27;
 
 inline bool aligned(const void* p, size_t a) { return ((uintptr_t)p & (a - 1)) == 0; }
 inline bool is_float_dtype(int dt) { return dt == SPH_F32 || dt == SPH_F16 || dt == SPH_BF16; }

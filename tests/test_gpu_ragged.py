@@ -1,0 +1,74 @@
+"""GPU parity where no 16-byte vector fits: widths that the vector does not divide and tensors that
+are only element-aligned, at the edges of the launch shapes (a run, a wave, the widest row held in
+registers, the cached / non-temporal bound).
+
+Norms: the fixed tests' bars (f32 <= 1e-5 relative, halves <= 1 ulp, LayerNorm the summation-order
+bound; the residual sum bit for bit). Reference: layernorm.rs:17-69, :75-106.
+"""
+import numpy as np
+import pytest
+import torch
+
+from helpers import (assert_bits16_equal, assert_bits_equal, assert_ulp16, check_layer_norm, max_rel, narrow_bits,
+                     to_np, widen)
+
+import sapient_amd.ops as ops
+
+pytestmark = pytest.mark.gpu
+DTYPES = [torch.float32, torch.float16, torch.bfloat16]
+DT_ID = lambda d: str(d).split(".")[-1]
+
+
+def _gen(shape, seed, dev, dtype, off=0, std=1.0, mean=0.0):
+    """Seeded values `off` elements into an allocation, so element-aligned only when off is odd."""
+    n = int(np.prod(shape))
+    g = torch.Generator(device=dev).manual_seed(seed)
+    return (torch.randn(n + off, generator=g, device=dev) * std + mean).to(dtype)[off:].view(shape)
+
+
+def _same(got, want32, dtype, orc, what):
+    if dtype == torch.float32:
+        assert_bits_equal(to_np(got), want32, what)
+    else:
+        assert_bits16_equal(to_np(got), narrow_bits(want32, dtype, orc), what)
+
+
+def _close(got, want32, orc, what):
+    if got.dtype == torch.float32:
+        assert max_rel(to_np(got), want32) <= 1e-5, what
+    else:
+        assert_ulp16(to_np(got), narrow_bits(want32, got.dtype, orc), got.dtype, 1, what)
+
+
+# One element; a run of 8 / 4 and one either side; one and two waves' spans; 16 waves at one and at two
+# runs per lane (f32 4096 / 8192, halves 8192 / 16384) and one past them; 65536 x 515: past the cached bound.
+@pytest.mark.parametrize("dtype", DTYPES, ids=DT_ID)
+@pytest.mark.parametrize("rows,dim,off", [(3, 1, 0), (5, 7, 0), (5, 9, 1), (4, 255, 0), (4, 257, 0), (3, 513, 3),
+                                          (700, 1025, 0), (2100, 1023, 0), (5, 4095, 0), (5, 4097, 1), (3, 8191, 0),
+                                          (3, 8193, 0), (2, 16383, 0), (2, 16385, 0), (65536, 515, 0), (9, 512, 1)])
+def test_ragged_norms(dev, orc, dtype, rows, dim, off):
+    print(f"case ragged norms {dtype} {rows}x{dim} offset {off}", flush=True)
+    x = _gen((rows, dim), 1, dev, dtype, off, mean=0.25)
+    r = _gen((rows, dim), 2, dev, dtype, off)
+    for wdt in {torch.float32, dtype}:
+        w, b = _gen((dim,), 3, dev, wdt, off, 0.1, 1.0), _gen((dim,), 4, dev, wdt, 0, 0.1)
+        w32, b32 = widen(w, orc), widen(b, orc)
+        y = ops.rms_norm(x, w, 1e-5)
+        ln = ops.layer_norm(x, w, b, 1e-5, out_dtype=torch.float32)
+        r2 = r.clone()
+        ya, r2 = ops.add_rms_norm(x, r2, w, 1e-5)
+        yt, st = ops.add_rms_norm(x, r, w, 1e-5, sum_out=torch.empty_like(r))
+        torch.cuda.synchronize()
+        assert torch.equal(st.view(torch.uint8), r2.view(torch.uint8))
+        # The rows at both ends and in the middle against the oracle: rows are independent.
+        pick = sorted({i for i in (0, 1, rows // 2, rows - 2, rows - 1) if 0 <= i < rows})
+        x32, r32 = widen(x[pick], orc), widen(r[pick], orc)
+        _close(y[pick], orc.rms_norm(x32, w32, 1e-5), orc, "rms_norm")
+        check_layer_norm(ln[pick], orc.layer_norm(x32, w32, b32, 1e-5), x32, w32, b32, orc, "layer_norm")
+        ref, ref_r = orc.add_rms_norm(x32, r32, w32, 1e-5)
+        _same(r2[pick], ref_r, dtype, orc, "residual")
+        _close(ya[pick], ref, orc, "add_rms_norm")
+        _close(yt[pick], ref, orc, "add_rms_norm_to")
+        # No row is skipped: every row's RMS is 1 where the weight is 1.
+        u = ops.rms_norm(x, None, 0.0, out_dtype=torch.float32)
+        assert (u.square().mean(-1) - 1).abs().max().item() < 1e-4
