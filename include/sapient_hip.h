@@ -304,13 +304,14 @@ int sph_kv_append(const void* src, int src_dtype, void* cache, int cache_dtype, 
  * returns SPH_ERANGE (the reference's "new tokens exceeds max cache size"),
  * cur_len > max_seq SPH_EINVAL; nothing is written then, nor when the append
  * itself would be rejected (its checks run before the shift). Types,
- * conversion and the Q8_0 layout are sph_kv_append's. The shift runs as two
- * in-place row-reversal passes (one launch each for n_kv <= 65535, more for
- * larger n_kv) and the append as one launch (more past 2^31 work items); the
- * rows moved by the shift are copied bit for bit, and the shift's rows past
+ * conversion and the Q8_0 layout are sph_kv_append's. The shift runs in place,
+ * in two launches per 65535 heads, and moves each kept row once where it is
+ * small against the rows a block holds (at least 31 f16 rows of 128), else
+ * twice; the append rides in the second launch where the cache's rows split
+ * into aligned 16-byte units, else it is a launch of its own. The rows moved
+ * by the shift are copied bit for bit, and the shift's rows past
  * cur_len - shift hold intermediate values until the append overwrites them.
- * The in-place shift moves every kept row twice; sph_kv_cache_update_into
- * moves it once, into a second buffer. */
+ * sph_kv_cache_update_into moves each kept row once, into a second buffer. */
 int sph_kv_cache_update(const void* src, int src_dtype, void* cache, int cache_dtype, int64_t n_kv, int64_t seq,
                         int64_t head_dim, int64_t max_seq, int64_t cur_len, int64_t* new_len, void* stream);
 

@@ -187,7 +187,9 @@ __global__ __launch_bounds__(kThreads) void kv_append_q8_0(const TS* __restrict_
 // rev(X) in the rows the append overwrites. A reversal is a set of disjoint
 // row swaps (row lo + j with row hi - 1 - j), so every thread swaps its units
 // on its own — no ordering between blocks, no scratch memory — and the kernel
-// boundary orders the two passes. Each pass reads and writes every row once
+// boundary orders the two passes; the second writes the new rows too where the cache's
+// rows split into 16-byte units (kv_reverse_append: f16 2 x 4096 x 64 7.7 -> 5.4 us, a launch
+// less). Shifts of a few rows move in windows instead (Windows). Each pass reads and writes every row once
 // (twice the bytes of a direct move) in whole rows, coalesced, over the whole
 // GPU; a direct in-place move must keep each column of a head in one block,
 // since a row is read by the row `shift` below it (16 bytes per row access,
@@ -227,6 +229,203 @@ int launch_reverse(void* cache, uint64_t n_heads, uint64_t row_bytes, uint64_t m
     return SPH_OK;
 }
 
+// The shift of a few rows (decode steps), each row moved once, in two launches. The rows [0, cur_len) of a
+// head are cut into windows.
+//  1. Every window's first `shift` rows (its slot) take the next window's: those are the rows that follow
+//     the window, and the rows a slot held are the ones that the window before it takes. (The first slot's
+//     rows are the dropped ones.)
+//  2. Every window rotates left by `shift`: its own rows move down and the slot's end it. The last window's
+//     end is the new rows' place.
+// A block holds all it moves in registers between its loads and its stores, so the in-place moves need no
+// order between blocks; only the two launches are ordered. HBM-bound: the second launch moves 33.5 MB in
+// 5.5-7.5 us, the first waits on memory once (1.6-2.7 us). A one-token update against the two reversal
+// passes and the append, in turn on one MI355X: f16 8 x 8192 x 128 12.6 -> 10.0 us, 32 x 4096 x 80 16.1 ->
+// 10.7, 8 x 32768 x 128 42.3 -> 25.3, 2 x 4096 x 64 8.7 -> 6.1; f32 8 x 8192 x 128 33.2 -> 16.6; Q8_0
+// 8 x 8192 x 128 11.2 -> 10.6. Non-temporal accesses cost 1-3 us.
+struct Windows {
+    uint32_t count, shift;
+    uint32_t step, rem;  // window c starts at row c * step + min(c, rem)
+    __device__ __forceinline__ uint32_t start(uint32_t c) const { return c * step + (c < rem ? c : rem); }
+};
+
+// Units per thread of a window (64 f16 rows of 128 a block); 2 and 8 measured 0.2-5 us slower.
+constexpr int kRotateUnits = 4;
+constexpr int kSlotThreads = 1024, kSlotUnits = 4;  // step 1 (256 or 512 threads: within 1 us either way)
+
+// Loads whose addresses another wave stores to after the barrier have to have arrived before it.
+__device__ __forceinline__ void loads_landed() {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+}
+
+// Step 1: a block owns `per_block` unit offsets of every slot of a head (count <= kSlotThreads * kSlotUnits).
+template <typename UT>
+__global__ __launch_bounds__(kSlotThreads) void kv_shift_slots(UT* cache, uint32_t upr, uint64_t max_seq, Windows w,
+                                                              uint32_t per_block) {
+    const uint32_t u0 = blockIdx.x * per_block, slot_units = w.shift * upr;
+    const uint32_t nu = slot_units - u0 < per_block ? slot_units - u0 : per_block;
+    const uint32_t n = (w.count - 1) * nu;
+    UT* base = cache + (uint64_t)blockIdx.y * max_seq * upr + u0;
+    UT v[kSlotUnits];
+#pragma unroll
+    for (int k = 0; k < kSlotUnits; ++k) {
+        const uint32_t i = (uint32_t)k * kSlotThreads + threadIdx.x;
+        const uint32_t c = i / nu;
+        if (i < n) v[k] = base[(uint64_t)w.start(c + 1) * upr + (i - c * nu)];
+    }
+    loads_landed();
+#pragma unroll
+    for (int k = 0; k < kSlotUnits; ++k) {
+        const uint32_t i = (uint32_t)k * kSlotThreads + threadIdx.x;
+        const uint32_t c = i / nu;
+        if (i < n) base[(uint64_t)w.start(c) * upr + (i - c * nu)] = v[k];
+    }
+}
+
+// Step 2, window blockIdx.x of head blockIdx.y: `append` writes the new rows over the last window's end,
+// once its rows are in registers (or is empty: a later launch writes them).
+template <typename UT, typename F>
+__device__ __forceinline__ void rotate_window(UT* head, uint32_t upr, const Windows& w, F&& append) {
+    const uint32_t start = w.start(blockIdx.x);
+    const uint32_t n = (w.start(blockIdx.x + 1) - start) * upr, sh = w.shift * upr;
+    const bool last = blockIdx.x == w.count - 1;
+    UT* base = head + (uint64_t)start * upr;
+    UT v[kRotateUnits];
+#pragma unroll
+    for (int k = 0; k < kRotateUnits; ++k) {
+        const uint32_t i = (uint32_t)k * kThreads + threadIdx.x;
+        if (i < n) v[k] = base[i];
+    }
+    loads_landed();
+#pragma unroll
+    for (int k = 0; k < kRotateUnits; ++k) {
+        const uint32_t i = (uint32_t)k * kThreads + threadIdx.x;
+        if (i < n && i >= sh) base[i - sh] = v[k];
+        if (i < sh && !last) base[i + n - sh] = v[k];
+    }
+    if (last) append();
+}
+
+template <typename UT>
+__global__ __launch_bounds__(kThreads) void kv_rotate_windows(UT* cache, uint32_t upr, uint64_t max_seq, Windows w) {
+    rotate_window(cache + (uint64_t)blockIdx.y * max_seq * upr, upr, w, [] {});
+}
+
+// Step 2 with the append: the last window's block writes the new rows on its own place, the blocks after it
+// those past cur_len.
+template <typename TS, typename TD>
+__global__ __launch_bounds__(kThreads) void kv_rotate_append(TD* cache, const TS* __restrict__ src, uint32_t upr,
+                                                             uint64_t max_seq, Windows w, uint64_t keep, uint32_t seq) {
+    constexpr int E = vec16<TD>::n;
+    TD* head = cache + (uint64_t)blockIdx.y * max_seq * upr * E;
+    const TS* s = src + (uint64_t)blockIdx.y * seq * upr * E;
+    TD* d = head + keep * upr * E;
+    auto append = [&](uint32_t i) { move_chunk<TS, TD, E>(s + (uint64_t)i * E, d + (uint64_t)i * E); };
+    if (blockIdx.x < w.count) {
+        rotate_window(reinterpret_cast<u32x4*>(head), upr, w, [&] {
+            for (uint32_t i = threadIdx.x; i < w.shift * upr; i += kThreads) append(i);
+        });
+    } else {
+        const uint32_t i = w.shift * upr + (blockIdx.x - w.count) * kThreads + threadIdx.x;
+        if (i < seq * upr) append(i);
+    }
+}
+
+// The window cut for a shift; count = 0 where it does not apply: a window has to hold twice the shift, so
+// that the slots' extra move stays well below the second move of every row that the reversal makes.
+inline Windows cut_windows(uint64_t cur_len, uint64_t shift, uint64_t upr) {
+    const uint64_t most = upr == 0 ? 0 : (uint64_t)kRotateUnits * kThreads / upr;  // rows a block holds
+    if (cur_len <= shift || cur_len > INT32_MAX || 2 * shift + 2 > most) return Windows{0, 0, 0, 0};
+    const uint64_t n = (cur_len + most - 1) / most;
+    if (n > kSlotThreads * kSlotUnits) return Windows{0, 0, 0, 0};
+    // n > 1: every window has at least cur_len / n > most / 2 > shift rows.
+    return Windows{(uint32_t)n, (uint32_t)shift, (uint32_t)(cur_len / n), (uint32_t)(cur_len % n)};
+}
+
+// The shift in windows; with TS also the append.
+template <typename UT, typename TS, typename TD>
+int shift_by_windows(void* cache, const TS* src, uint64_t n_heads, uint64_t upr, uint64_t seq, uint64_t max_seq,
+                     uint64_t keep, const Windows& w, hipStream_t stream) {
+    constexpr uint64_t kMaxY = 65535;  // heads per launch (grid y)
+    for (uint64_t h0 = 0; h0 < n_heads; h0 += kMaxY) {
+        const unsigned nh = (unsigned)(n_heads - h0 < kMaxY ? n_heads - h0 : kMaxY);
+        UT* base = static_cast<UT*>(cache) + h0 * max_seq * upr;
+        int st = SPH_OK;
+        if (w.count > 1) {
+            const uint32_t slot_units = w.shift * (uint32_t)upr;
+            uint32_t per_block = (uint32_t)(kSlotThreads * kSlotUnits) / (w.count - 1);
+            if (per_block > slot_units) per_block = slot_units;
+            st = launch(kv_shift_slots<UT>, dim3((slot_units + per_block - 1) / per_block, nh), kSlotThreads, stream, base,
+                        (uint32_t)upr, max_seq, w, per_block);
+            if (st != SPH_OK) return st;
+        }
+        if constexpr (!std::is_same<TS, void>::value) {
+            constexpr uint64_t E = vec16<TD>::n;
+            const uint64_t past = (seq - w.shift) * upr;  // units of new rows past cur_len
+            st = launch(kv_rotate_append<TS, TD>, dim3(w.count + (unsigned)((past + kThreads - 1) / kThreads), nh), kThreads,
+                        stream, reinterpret_cast<TD*>(base), src + h0 * seq * upr * E, (uint32_t)upr, max_seq, w, keep,
+                        (uint32_t)seq);
+        } else {
+            st = launch(kv_rotate_windows<UT>, dim3(w.count, nh), kThreads, stream, base, (uint32_t)upr, max_seq, w);
+        }
+        if (st != SPH_OK) return st;
+    }
+    return SPH_OK;
+}
+
+// Second reversal pass (the whole of [0, n)) with the append: a row that the pass would leave from `keep`
+// on is written from src by the thread that has read it; rows [n, keep + seq) follow the pairs.
+template <typename TS, typename TD>
+__global__ __launch_bounds__(kThreads) void kv_reverse_append(TD* cache, const TS* __restrict__ src, uint32_t upr,
+                                                              uint64_t max_seq, uint32_t n, uint32_t keep, uint32_t seq,
+                                                              uint32_t items) {
+    constexpr int E = vec16<TD>::n;
+    const uint32_t i = blockIdx.x * (uint32_t)kThreads + threadIdx.x;
+    if (i >= items) return;
+    const uint32_t j = i / upr, u = i - j * upr;
+    TD* head = cache + (uint64_t)blockIdx.y * max_seq * upr * E + (uint64_t)u * E;
+    const TS* s = src + (uint64_t)blockIdx.y * seq * upr * E + (uint64_t)u * E;
+    auto row = [&](uint32_t r) { return reinterpret_cast<u32x4*>(head + (uint64_t)r * upr * E); };
+    auto append = [&](uint32_t r) {
+        move_chunk<TS, TD, E>(s + (uint64_t)(r - keep) * upr * E, head + (uint64_t)r * upr * E);
+    };
+    const uint32_t pairs = (n + 1) / 2;
+    if (j >= pairs) {
+        append(n + (j - pairs));
+        return;
+    }
+    const uint32_t b = n - 1 - j;  // j itself for the middle row of an odd n
+    const u32x4 va = *row(j), vb = *row(b);
+    if (j < keep) *row(j) = vb;
+    else append(j);
+    if (b == j) return;
+    if (b < keep) *row(b) = va;
+    else append(b);
+}
+
+// Shift and append of a float cache whose rows split into 16-byte units.
+template <typename TS, typename TD>
+int shift_append(const void* src, void* cache, uint64_t n_heads, uint64_t hd, uint64_t seq, uint64_t max_seq,
+                 uint64_t shift, uint64_t cur_len, hipStream_t stream) {
+    constexpr uint64_t E = vec16<TD>::n;
+    const uint64_t upr = hd / E, keep = cur_len - shift;
+    const TS* s = static_cast<const TS*>(src);
+    const Windows w = cut_windows(cur_len, shift, upr);
+    if (w.count > 0) return shift_by_windows<u32x4, TS, TD>(cache, s, n_heads, upr, seq, max_seq, keep, w, stream);
+    int st = launch_reverse<u32x4>(cache, n_heads, hd * sizeof(TD), max_seq, shift, cur_len, stream);
+    if (st != SPH_OK) return st;
+    constexpr uint64_t kMaxY = 65535;  // heads per launch (grid y)
+    const uint64_t items = ((cur_len + 1) / 2 + (keep + seq - cur_len)) * upr;
+    for (uint64_t h0 = 0; h0 < n_heads; h0 += kMaxY) {
+        const unsigned nh = (unsigned)(n_heads - h0 < kMaxY ? n_heads - h0 : kMaxY);
+        st = launch(kv_reverse_append<TS, TD>, dim3((unsigned)((items + kThreads - 1) / kThreads), nh), kThreads, stream,
+                    static_cast<TD*>(cache) + h0 * max_seq * hd, s + h0 * seq * hd, (uint32_t)upr, max_seq,
+                    (uint32_t)cur_len, (uint32_t)keep, (uint32_t)seq, (uint32_t)items);
+        if (st != SPH_OK) return st;
+    }
+    return SPH_OK;
+}
+
 // The two passes, with the widest unit the row width and the cache's alignment allow.
 // The second pass covers more rows than the first, so checking its item count
 // before either launch means a rejected shift leaves the cache untouched.
@@ -235,6 +434,9 @@ int shift_window(void* cache, uint64_t n_heads, uint64_t row_bytes, uint64_t max
                  uint64_t cur_len, hipStream_t stream) {
     const uint64_t upr = row_bytes / sizeof(UT);
     if (upr > UINT32_MAX || cur_len / 2 * upr > UINT32_MAX - kThreads) return SPH_EINVAL;
+    const Windows w = cut_windows(cur_len, shift, upr);
+    if (w.count > 0)
+        return shift_by_windows<UT, void, void>(cache, nullptr, n_heads, upr, 0, max_seq, cur_len - shift, w, stream);
     const int st = launch_reverse<UT>(cache, n_heads, row_bytes, max_seq, shift, cur_len, stream);
     if (st != SPH_OK) return st;
     return launch_reverse<UT>(cache, n_heads, row_bytes, max_seq, 0, cur_len, stream);
@@ -423,6 +625,22 @@ extern "C" int sph_kv_cache_update(const void* src, int src_dtype, void* cache, 
         if (cache == nullptr) return SPH_EINVAL;
         const uint64_t row_bytes = q8 ? (uint64_t)head_dim / 32 * 34 : (uint64_t)head_dim * sph::dtype_size(cache_dtype);
         int st;
+        // Float caches whose rows split into 16-byte units: the append rides in the shift's last launch.
+        if (!q8 && row_bytes % 16 == 0 && sph::aligned(cache, 16)) {
+            const uint64_t e = 16 / sph::dtype_size(cache_dtype), src_access = e * sph::dtype_size(src_dtype);
+            if (sph::aligned(src, src_access < 16 ? src_access : 16) &&
+                ((uint64_t)cur_len / 2 + 1 + (uint64_t)seq) * ((uint64_t)head_dim / e) <= UINT32_MAX - sph::kThreads) {
+                st = sph::with_float_type(src_dtype, [&](auto ts) -> int {
+                    using TS = decltype(ts);
+                    return sph::with_float_type(cache_dtype, [&](auto td) -> int {
+                        using TD = decltype(td);
+                        return sph::shift_append<TS, TD>(src, cache, n_kv, head_dim, seq, max_seq, shift, cur_len, s);
+                    });
+                });
+                if (st == SPH_OK) *new_len = max_seq;
+                return st;
+            }
+        }
         if (row_bytes % 16 == 0 && sph::aligned(cache, 16))
             st = sph::shift_window<sph::u32x4>(cache, n_kv, row_bytes, max_seq, shift, cur_len, s);
         else if (row_bytes % 8 == 0 && sph::aligned(cache, 8))

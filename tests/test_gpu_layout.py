@@ -397,3 +397,36 @@ def test_kv_cache_update_into_rejects_bad_arguments(dev):
     assert L.sph_kv_cache_update_into(x, 0, c, o, 8, 2, 1, 16, 8, 8, a, s) == EINVAL     # Q8_0 at hd 16
     torch.cuda.synchronize()
     assert n.value == -7 and torch.equal(cache, before) and torch.equal(out, out_before)
+
+
+# In-place slides across the launch forms. In windows: one window and two, the largest shift a window takes and
+# one more (f16 rows of 128: 31; f32: 15), more new rows than the shift, rows of each unit width, many heads.
+# By reversal with the append: odd and even cur_len, a shift past the middle. Q8_0: the append on its own.
+@pytest.mark.parametrize("cdtype,n_kv,hd,max_seq,cur_len,seq", [
+    (torch.float16, 2, 128, 64, 64, 1), (torch.float16, 2, 128, 65, 65, 1), (torch.bfloat16, 3, 64, 34, 33, 2),
+    (torch.float32, 2, 8, 40, 37, 30), (torch.float32, 1, 4, 9, 9, 5), (torch.float16, 2, 40, 1000, 995, 20),
+    (torch.float16, 32, 128, 4096, 4094, 900), (torch.bfloat16, 8, 128, 12345, 12345, 31),
+    (torch.float32, 8, 128, 8191, 8190, 9), (torch.float32, 2, 128, 2000, 2000, 15), (torch.float16, 3000, 64, 60, 60, 1),
+    (torch.float16, 2, 128, 300, 300, 32), (torch.bfloat16, 2, 128, 301, 300, 41), (torch.float32, 2, 128, 64, 61, 50),
+    (torch.float32, 2, 128, 501, 501, 16), (torch.float16, 2, 128, 50, 50, 50),
+    (torch.uint8, 32, 128, 5000, 5000, 1), (torch.uint8, 3, 96, 701, 700, 3), (torch.uint8, 2, 64, 300, 300, 100)])
+def test_kv_cache_update_in_place_forms(dev, cdtype, n_kv, hd, max_seq, cur_len, seq):
+    print(f"case kv_cache_update forms {cdtype} {n_kv}x{hd} max {max_seq} cur {cur_len} seq {seq}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(n_kv + hd)
+    src = torch.randn((n_kv, seq, hd), generator=g, device=dev)
+    if cdtype == torch.uint8:
+        cache = torch.randint(0, 256, (n_kv, max_seq, hd // 32 * 34), generator=g, device=dev, dtype=torch.uint8)
+        new = torch.zeros((n_kv, seq, hd // 32 * 34), device=dev, dtype=torch.uint8)
+        ops.kv_append(src, new, 0)  # checked against the oracle above
+    else:
+        cache = torch.randn((n_kv, max_seq, hd), generator=g, device=dev).to(cdtype)
+        new = src.to(cdtype)
+    shift = cur_len + seq - max_seq
+    want = torch.cat([cache[:, shift:cur_len], new], 1)
+    guard = torch.full((4096,), 7, device=dev, dtype=cache.dtype)  # the bytes after the cache
+    both = torch.cat([cache.reshape(-1), guard])
+    view = both[:cache.numel()].view(cache.shape)
+    assert ops.kv_cache_update(src, view, cur_len) == max_seq
+    torch.cuda.synchronize()
+    assert torch.equal(view.view(torch.uint8), want.contiguous().view(torch.uint8))
+    assert torch.equal(both[cache.numel():], guard)
