@@ -139,43 +139,63 @@ int launch_move(const void* src, void* dst, uint64_t rows, uint64_t hd, RowMap m
     return SPH_OK;
 }
 
-// Q8_0 cache: one thread per 32-element block of a (head, token) row, the
-// quantizer of the reference's quantized KV cache
+// Q8_0 cache: the quantizer of the reference's quantized KV cache
 // (crates/sapient-models/src/forward/common.rs:336-348, the same steps as
-// quant.rs:223-235): amax over the block (NaN skipped, as f32::max folds),
-// scale = amax / 127 in f32, d = f16(scale), q = clamp(round(v · 1/scale),
-// ±127) with round half away from zero and NaN → 0 (the `as i8` cast), and 0
-// throughout for an all-zero block. Row layout: head_dim / 32 blocks of
-// 34 bytes (f16 d, 32 × i8), rows of a head at positions 0 .. max_seq - 1.
+// quant.rs:223-235) over each 32-element block of a (head, token) row: amax
+// (NaN skipped, as f32::max folds), scale = amax / 127 in f32, d = f16(scale),
+// q = clamp(round(v · 1/scale), ±127) with round half away from zero and NaN →
+// 0 (the `as i8` cast), and 0 throughout for an all-zero block. Row layout:
+// head_dim / 32 blocks of 34 bytes (f16 d, 32 × i8), rows of a head at
+// positions 0 .. max_seq - 1.
+// A block is read by kQ8Lanes neighbouring lanes, which share the amax through
+// DPP moves: a wave's accesses are contiguous, where one thread per block
+// walked its 128 bytes alone, 64 lanes 128 bytes apart.
+// Bound by the quantizer's ~30 VALU operations per four elements as much as by
+// its bytes: at f32 8 x 2048 x 128 (10.6 MB) 4.0 us one thread per block, 3.0
+// with four lanes, 3.2 with two, 3.9 with eight (each lane divides twice), 4.3
+// with eight and the packed blocks leaving through LDS in 16-byte stores; a
+// decode step (8 x 1 x 128) 2.7 -> 1.9.
+// items / kQ8Lanes / bpr rows from token s0 of the first head of src and cache.
+constexpr uint32_t kQ8Lanes = 4;
+
+// round(t), half away from zero, of |t| <= 127.5 (f32's predecessor of 1/2 is added, so that no sum
+// below the next integer rounds up to it), clamped to ±127; NaN → 0.
+__device__ __forceinline__ uint32_t q8_byte(float t) {
+    t = t == t ? fminf(fmaxf(t, -127.0f), 127.0f) : 0.0f;
+    return (uint32_t)(int32_t)(t + __builtin_copysignf(0x1.fffffep-2f, t)) & 0xFFu;
+}
+
 template <typename TS>
 __global__ __launch_bounds__(kThreads) void kv_append_q8_0(const TS* __restrict__ src, uint8_t* __restrict__ cache,
-                                                           uint64_t blocks, uint32_t bpr, uint32_t seq,
-                                                           uint32_t max_seq, uint64_t pos) {
-    const uint64_t k = (uint64_t)blockIdx.x * kThreads + threadIdx.x;
-    if (k >= blocks) return;
-    const uint64_t row = k / bpr;                // source row h · seq + s
-    const uint32_t blk = (uint32_t)(k - row * bpr);
-    const uint64_t h = row / seq, s = row - h * seq;
-    float v[32];
-    load_f32<TS, 32>(src + row * (uint64_t)bpr * 32 + (uint64_t)blk * 32, v);
+                                                           uint32_t items, uint32_t bpr, uint32_t seq,
+                                                           uint32_t max_seq, uint64_t pos, uint32_t s0) {
+    constexpr uint32_t L = kQ8Lanes;
+    constexpr int V = 32 / (int)L;  // values per lane
+    const uint32_t i = blockIdx.x * (uint32_t)kThreads + threadIdx.x;
+    if (i >= items) return;         // items is a multiple of L: a block's lanes leave together
+    const uint32_t k = i / L, lane = i % L;
+    const uint32_t r = k / bpr, blk = k - r * bpr;
+    const uint32_t row = s0 + r;    // source row h · seq + s (below 2^32: see the launch)
+    const uint32_t h = row / seq, s = row - h * seq;
+    float v[V];
+    load_f32<TS, V>(src + ((uint64_t)row * bpr + blk) * 32 + lane * V, v);
     float amax = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 32; ++i) amax = fmaxf(amax, fabsf(v[i]));
+    for (int e = 0; e < V; ++e) amax = fmaxf(amax, fabsf(v[e]));
+    amax = fmaxf(amax, dpp_mov<0xb1>(amax));  // quad_perm [1,0,3,2]
+    amax = fmaxf(amax, dpp_mov<0x4e>(amax));  // quad_perm [2,3,0,1]
     const float scale = amax / 127.0f;
     const float inv = scale > 0.0f ? 1.0f / scale : 0.0f;
-    uint8_t* out = cache + ((h * max_seq + pos + s) * (uint64_t)bpr + blk) * 34;  // 2-byte aligned
-    uint16_t* o16 = reinterpret_cast<uint16_t*>(out);
-    o16[0] = narrow<f16>(scale).bits;
+    uint8_t* out = cache + (((uint64_t)h * max_seq + pos + s) * bpr + blk) * 34;  // 2-byte aligned
+    if (lane == 0) *reinterpret_cast<uint16_t*>(out) = narrow<f16>(scale).bits;
+    typedef uint32_t words __attribute__((ext_vector_type(V / 4)));
+    typedef words words_at2 __attribute__((aligned(2)));
+    words q;
 #pragma unroll
-    for (int i = 0; i < 32; i += 2) {
-        int8_t q[2];
-#pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const float r = roundf(v[i + j] * inv);  // half away from zero
-            q[j] = r != r ? (int8_t)0 : (int8_t)fminf(fmaxf(r, -127.0f), 127.0f);
-        }
-        o16[1 + i / 2] = (uint16_t)((uint8_t)q[0] | ((uint16_t)(uint8_t)q[1] << 8));
-    }
+    for (int w = 0; w < V / 4; ++w)
+        q[w] = q8_byte(v[4 * w] * inv) | q8_byte(v[4 * w + 1] * inv) << 8 | q8_byte(v[4 * w + 2] * inv) << 16 |
+               q8_byte(v[4 * w + 3] * inv) << 24;
+    *reinterpret_cast<words_at2*>(out + 2 + lane * V) = q;
 }
 
 // Sliding-window shift of a KV cache (the trait path's update_kv_cache,
@@ -587,13 +607,28 @@ extern "C" int sph_kv_append(const void* src, int src_dtype, void* cache, int ca
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (q8) {
         const uint64_t bpr = (uint64_t)head_dim / 32;
-        const uint64_t blocks = rows * bpr;
         return sph::with_float_type(src_dtype, [&](auto ts) -> int {
             using TS = decltype(ts);
-            const dim3 grid((unsigned)((blocks + sph::kThreads - 1) / sph::kThreads));
-            return sph::launch(sph::kv_append_q8_0<TS>, grid, sph::kThreads, s, static_cast<const TS*>(src),
-                               static_cast<uint8_t*>(cache), blocks, (uint32_t)bpr, (uint32_t)seq, (uint32_t)max_seq,
-                               (uint64_t)pos);
+            // Launches of fewer than 2^32 lanes: whole heads, or runs of one head's rows.
+            constexpr uint64_t kItems = (uint64_t)1 << 31;
+            const uint64_t row_items = bpr * sph::kQ8Lanes, head_items = row_items * (uint64_t)seq;
+            const bool heads = head_items <= kItems;
+            const uint64_t step_h = heads ? kItems / head_items : 1, step_s = heads ? (uint64_t)seq : kItems / row_items;
+            if (step_s == 0) return SPH_EINVAL;
+            for (uint64_t h0 = 0; h0 < (uint64_t)n_kv; h0 += step_h) {
+                const uint64_t nh = (uint64_t)n_kv - h0 < step_h ? (uint64_t)n_kv - h0 : step_h;
+                for (uint64_t s0 = 0; s0 < (uint64_t)seq; s0 += step_s) {
+                    const uint64_t ns = (uint64_t)seq - s0 < step_s ? (uint64_t)seq - s0 : step_s;
+                    const uint32_t items = (uint32_t)(nh * ns * row_items);
+                    const int st = sph::launch(
+                        sph::kv_append_q8_0<TS>, dim3((items + sph::kThreads - 1) / sph::kThreads), sph::kThreads, s,
+                        static_cast<const TS*>(src) + h0 * (uint64_t)seq * (uint64_t)head_dim,
+                        static_cast<uint8_t*>(cache) + h0 * (uint64_t)max_seq * bpr * 34, items, (uint32_t)bpr,
+                        (uint32_t)seq, (uint32_t)max_seq, (uint64_t)pos, (uint32_t)s0);
+                    if (st != SPH_OK) return st;
+                }
+            }
+            return SPH_OK;
         });
     }
     const sph::RowMap m{(uint32_t)seq, (uint32_t)max_seq, (uint64_t)pos};
