@@ -41,6 +41,7 @@ namespace sph {
 namespace {
 
 constexpr int kThreads = 256;
+constexpr int kWave = 64;
 constexpr int kMaxHalf = 256;  // rotary_dim <= 512
 
 struct DenTable {
@@ -75,7 +76,7 @@ __device__ __forceinline__ const uint32_t* stage_inv_pio4(uint32_t (&tab)[24]) {
 // or single elements when the run is narrower than a word or ELEM asks for
 // element accesses: rows only element-aligned), so that a batch of rows can be
 // in flight while the previous batch is rotated and stored.
-template <typename T, int L, bool ELEM = false>
+template <typename T, int L, bool ELEM = false, bool NT = true>
 struct RawRun {
     static constexpr bool kWords = !ELEM && (L * (int)sizeof(T)) % 4 == 0;
     uint32_t w[kWords ? words_of<T, L>::n : 1];
@@ -83,7 +84,7 @@ struct RawRun {
 
     __device__ __forceinline__ void load(const T* p) {
         if constexpr (kWords) {
-            load_words<T, L, true>(p, w);
+            load_words<T, L, NT>(p, w);
         } else {
 #pragma unroll
             for (int i = 0; i < L; ++i) e[i] = p[i];
@@ -99,10 +100,10 @@ struct RawRun {
     }
 };
 
-template <typename T, int L, bool ELEM = false>
+template <typename T, int L, bool ELEM = false, bool NT = true>
 __device__ __forceinline__ void store_run(T* p, const float (&v)[L]) {
     if constexpr (!ELEM && (L * (int)sizeof(T)) % 4 == 0) {
-        store_f32<T, L, true>(p, v);
+        store_f32<T, L, NT>(p, v);
     } else {
 #pragma unroll
         for (int i = 0; i < L; ++i) p[i] = narrow<T>(v[i]);
@@ -347,183 +348,233 @@ __global__ __launch_bounds__(kThreads) void rope_kernel(T* q, int nq, T* k, int 
     }
 }
 
+// Everything a fused launch reads, by value (den, where the angles are evaluated, by lane).
+template <typename T, typename TC>
+struct RopeKvArgs {
+    const T* q;
+    T* qo;
+    const T* k;
+    const T* v;
+    TC* kc;
+    TC* vc;
+    const int32_t* pos;
+    const void* bias[3];  // of q, k, v; each may be null
+    int bias_dt;
+    int nq, nkv;
+    int64_t seq, max_seq;
+    int head_dim, half;
+    int lanes, toks, heads;  // lanes per row; a block's tokens, and its heads per pass
+    int h_first;             // the launch's first head
+    float pos_scale;
+    int32_t* bad;
+    const float* ang;
+    bool ang_by_pos;
+    DenTable den;
+};
+
+constexpr int kMaxBlockAngles = 256;  // a block's tokens times pairs
+
+// A thread's share of a row, as it sits in memory: P pairs, in two runs of P elements at i0 and
+// half + i0 (NEOX) or one of 2P at 2 i0 (interleaved). In f32, f holds the runs one after the other.
+template <typename T, int P, bool INTERLEAVED, bool NT>
+struct PairRuns {
+    static constexpr int R = INTERLEAVED ? 1 : 2, L = INTERLEAVED ? 2 * P : P;
+    RawRun<T, L, false, NT> run[R];
+    __device__ __forceinline__ static int at(int r, int i0, int half) { return INTERLEAVED ? 2 * i0 : i0 + r * half; }
+    __device__ __forceinline__ void load(const T* row, int i0, int half) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) run[r].load(row + at(r, i0, half));
+    }
+    __device__ __forceinline__ void to_f32(float (&f)[2 * P]) const {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            float t[L];
+            run[r].to_f32(t);
+#pragma unroll
+            for (int j = 0; j < L; ++j) f[r * L + j] = t[j];
+        }
+    }
+    template <typename TR>
+    __device__ __forceinline__ static void store(TR* row, int i0, int half, const float (&f)[2 * P]) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            float t[L];
+#pragma unroll
+            for (int j = 0; j < L; ++j) t[j] = f[r * L + j];
+            store_run<TR, L, false, NT>(row + at(r, i0, half), t);
+        }
+    }
+};
+
+// N consecutive bias values (of any float type) as f32; the launch checked their alignment.
+template <int N>
+__device__ __forceinline__ void load_bias(const void* p, int dt, int at, float (&b)[N]) {
+    if (dt == SPH_F32) {
+        load_f32<float, N>(static_cast<const float*>(p) + at, b);
+    } else if constexpr (N % 2 == 0) {
+        if (dt == SPH_F16) load_f32<f16, N>(static_cast<const f16*>(p) + at, b);
+        else load_f32<bf16, N>(static_cast<const bf16*>(p) + at, b);
+    } else {
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+            b[i] = dt == SPH_F16 ? widen(static_cast<const f16*>(p)[at + i]) : widen(static_cast<const bf16*>(p)[at + i]);
+    }
+}
+
 // Fused decode step: heads [0, nq) are q rows, rotated and written to qo
 // heads-major; heads [nq, nq + nkv) rotate the k row and write it, plus the v
 // row, to cache row (h, positions[s]). batch = 1 and rotary_dim = head_dim, so
 // a thread's P pairs and the pairs of its lane neighbours cover every channel
 // of the row. TM: q, k and v are read token-major [seq, heads, head_dim] (the
 // projections' layout) instead of heads-major; without TM, qo == q (in place).
-template <typename T, typename TC, typename TB, int P, bool INTERLEAVED, bool TM>
-__global__ __launch_bounds__(kThreads) void rope_kv_kernel(const T* q, T* qo, int nq, const T* __restrict__ k,
-                                                           const T* __restrict__ v, int nkv,
-                                                           const int32_t* __restrict__ pos, int64_t seq, int head_dim,
-                                                           int half, int lanes_per_tok, int toks_per_block,
-                                                           int heads_per_group, float pos_scale, TC* kc, TC* vc,
-                                                           int64_t max_seq, int32_t* bad_pos_flag, const TB* bq,
-                                                           const TB* bk, const TB* bv, DenTable den,
-                                                           const float* __restrict__ ang, bool ang_by_pos) {
+// A block covers a few tokens by U passes of a few heads. Its angles (tokens x
+// pairs, at most one per thread) are evaluated once, into LDS, while the rows'
+// loads are in flight, and shared by all its heads: glibc's sincos in double
+// arithmetic is the long pole of a launch that would otherwise wait on memory
+// once. Threads take the angles pair-major, so a wave's are of one size and
+// only waves of low pairs run the large-argument reduction.
+template <typename T, typename TC, int P, bool INTERLEAVED, bool TM, int U, bool BIAS, bool NT>
+__global__ __launch_bounds__(kThreads) void rope_kv_kernel(RopeKvArgs<T, TC> a) {
     __shared__ uint32_t inv_pio4[24];
-    const int tib = threadIdx.x / lanes_per_tok;
-    const int lit = threadIdx.x - tib * lanes_per_tok;
-    const int64_t s = (int64_t)blockIdx.x * toks_per_block + tib;
-    const bool active = tib < toks_per_block && s < seq;
+    __shared__ float cs_s[kMaxBlockAngles], sn_s[kMaxBlockAngles];
+    const int tid = threadIdx.x;
+    const int rho = tid / a.lanes, lit = tid - rho * a.lanes;
+    const int tl = TM ? rho / a.heads : rho % a.toks;  // neighbouring rows in memory: heads (TM), else tokens
+    const int hl = TM ? rho - tl * a.heads : rho / a.toks;
+    const int64_t s0 = (int64_t)blockIdx.x * a.toks, s = s0 + tl;
+    const bool active = rho < a.toks * a.heads && s < a.seq;
+    const int h0 = a.h_first + (int)blockIdx.y * a.heads * U + hl, H = a.nq + a.nkv;
     const int i0 = lit * P;
-    // Element offsets of this thread's two runs of P elements within a row.
-    const int a0 = INTERLEAVED ? 2 * i0 : i0;
-    const int a1 = INTERLEAVED ? 2 * i0 + P : i0 + half;
-    const int h_begin = blockIdx.y * heads_per_group;
-    int h_end = h_begin + heads_per_group;
-    if (h_end > nq + nkv) h_end = nq + nkv;
+    using Runs = PairRuns<T, P, INTERLEAVED, NT>;
+
+    const bool eval = a.ang == nullptr;
+    constexpr bool kOwn = P == 1;  // a thread's one angle: no exchange (3 tokens of 14 + 2 x 64: 2.87 -> 2.66 us)
+    uint32_t tab_word = 0;
+    if (eval && tid < 24) tab_word = kInvPio4.w[tid];
+    // Angle number tid of the block.
+    const int pair = eval && !kOwn ? tid / a.toks : 0, tk = tid - pair * a.toks;
+    const bool has_angle = eval && !kOwn && pair < a.half;
+    float den = 1.0f;
+    if (kOwn && eval && active) den = a.den.v[i0];
+    int32_t apos = 0;
+    if (has_angle) {
+        den = a.den.v[pair];
+        if (s0 + tk < a.seq) apos = a.pos[s0 + tk];
+    }
+    int32_t ps = 0;
+    if (active) ps = a.pos[s];
 
     // Row (head h, token s) of a [heads, seq, hd] (or, TM, [seq, heads, hd]) tensor.
     auto row_of = [&](const T* base, int heads, int h) {
-        return base + (TM ? (size_t)s * (size_t)heads + (size_t)h : (size_t)h * (size_t)seq + (size_t)s) *
-                          (size_t)head_dim;
+        return base + (TM ? (size_t)s * (size_t)heads + (size_t)h : (size_t)h * (size_t)a.seq + (size_t)s) *
+                          (size_t)a.head_dim;
     };
-    // Row values with the bias of their channels added (y + b in f32, then
-    // stored in the activation type before RoPE reads it: round through T).
-    auto load_row = [&](const T* row, const TB* bias, float (&u0)[P], float (&u1)[P]) {
-        if constexpr (!INTERLEAVED) {
-            load_f32<T, P, true>(row + a0, u0);
-            load_f32<T, P, true>(row + a1, u1);
-        } else {
-            float x[2 * P];
-            load_f32<T, 2 * P, true>(row + a0, x);
+    Runs x[U], w[U];  // the q or k row, and the v row
+    float xb[BIAS ? U : 1][2 * P], wb[BIAS ? U : 1][2 * P];  // their biases
+    auto bias_of = [&](int which, int h, float (&b)[2 * P]) {
+        if (a.bias[which] == nullptr) return;
 #pragma unroll
-            for (int j = 0; j < P; ++j) {
-                u0[j] = x[2 * j];
-                u1[j] = x[2 * j + 1];
-            }
+        for (int r = 0; r < Runs::R; ++r) {
+            float t[Runs::L];
+            load_bias<Runs::L>(a.bias[which], a.bias_dt, h * a.head_dim + Runs::at(r, i0, a.half), t);
+#pragma unroll
+            for (int j = 0; j < Runs::L; ++j) b[r * Runs::L + j] = t[j];
         }
-        if (bias != nullptr) {
-            float b0[P], b1[P];
-            if constexpr (!INTERLEAVED) {
-                load_f32<TB, P>(bias + a0, b0);
-                load_f32<TB, P>(bias + a1, b1);
-            } else {
-                float b[2 * P];
-                load_f32<TB, 2 * P>(bias + a0, b);
+    };
 #pragma unroll
-                for (int j = 0; j < P; ++j) {
-                    b0[j] = b[2 * j];
-                    b1[j] = b[2 * j + 1];
+    for (int u = 0; u < U; ++u) {
+        const int h = h0 + u * a.heads;
+        if (active && h < H) {
+            const T* r = h < a.nq ? row_of(a.q, a.nq, h) : row_of(a.k, a.nkv, h - a.nq);
+            x[u].load(r, i0, a.half);
+            if (h >= a.nq) w[u].load(row_of(a.v, a.nkv, h - a.nq), i0, a.half);
+            if constexpr (BIAS) {
+                if (h < a.nq) {
+                    bias_of(0, h, xb[u]);
+                } else {
+                    bias_of(1, h - a.nq, xb[u]);
+                    bias_of(2, h - a.nq, wb[u]);
                 }
             }
-#pragma unroll
-            for (int j = 0; j < P; ++j) {
-                u0[j] = widen(narrow<T>(u0[j] + b0[j]));
-                u1[j] = widen(narrow<T>(u1[j] + b1[j]));
-            }
-        }
-    };
-
-    // The position and the first head's rows need neither the angle nor the
-    // table: they are issued before the table is staged, so the block waits
-    // on memory once instead of three times (what a one-token decode step
-    // costs is mostly these latencies).
-    int32_t ps = 0;
-    float x0[P], x1[P], v0[P], v1[P];
-    // A head's input rows: q (heads < nq), or k and v. (A macro: a lambda taking
-    // these arrays by reference left them in scratch memory for P = 1.)
-#define SPH_LOAD_HEAD(hh)                                                                         \
-    do {                                                                                          \
-        if ((hh) < nq) {                                                                          \
-            load_row(row_of(q, nq, (hh)), bq ? bq + (size_t)(hh) * head_dim : nullptr, x0, x1);   \
-        } else {                                                                                  \
-            const int h_ = (hh) - nq;                                                             \
-            load_row(row_of(k, nkv, h_), bk ? bk + (size_t)h_ * head_dim : nullptr, x0, x1);      \
-            load_row(row_of(v, nkv, h_), bv ? bv + (size_t)h_ * head_dim : nullptr, v0, v1);      \
-        }                                                                                         \
-    } while (0)
-    float cs[P], sn[P];
-    if (ang != nullptr && !ang_by_pos) {
-        // Angles supplied per (token, pair) as (cos, sin): requested with the
-        // position and the rows, so the step waits on memory once and computes
-        // no sin/cos (the whole block takes this branch; no barrier follows).
-        if (!active) return;
-        ps = pos[s];
-        const float* a = ang + 2 * ((size_t)s * (size_t)half + (size_t)i0);
-#pragma unroll
-        for (int j = 0; j < P; ++j) {
-            cs[j] = a[2 * j];
-            sn[j] = a[2 * j + 1];
-        }
-        if (h_begin < h_end) SPH_LOAD_HEAD(h_begin);
-    } else if (ang != nullptr) {
-        // Angles read from row pos[s] of a per-position table of max_seq rows
-        // (the first head's rows are requested before the position is waited
-        // on). A position outside [0, max_seq) reads no row: q is rotated by
-        // angle 0 (cos 1, sin 0), the caches are left alone and the flag set.
-        if (!active) return;
-        ps = pos[s];
-        if (h_begin < h_end) SPH_LOAD_HEAD(h_begin);
-        const bool in_table = ps >= 0 && (int64_t)ps < max_seq;
-        const float* a = ang + 2 * ((size_t)(in_table ? ps : 0) * (size_t)half + (size_t)i0);
-#pragma unroll
-        for (int j = 0; j < P; ++j) {
-            cs[j] = in_table ? a[2 * j] : 1.0f;
-            sn[j] = in_table ? a[2 * j + 1] : 0.0f;
-        }
-    } else {
-        if (active) {
-            ps = pos[s];
-            if (h_begin < h_end) SPH_LOAD_HEAD(h_begin);
-        }
-        const uint32_t* tab = stage_inv_pio4(inv_pio4);
-        if (!active) return;
-        const float p = (float)ps / pos_scale;
-#pragma unroll
-        for (int j = 0; j < P; ++j) {
-            const float freq = p / den.v[i0 + j];
-            glibc_sincosf_tab(freq, tab, &sn[j], &cs[j]);
         }
     }
-    const bool pos_ok = ps >= 0 && (int64_t)ps < max_seq;
-    if (!pos_ok && bad_pos_flag != nullptr && lit == 0 && blockIdx.y == 0) *bad_pos_flag = 1;
 
-    auto put = [&](auto* row, const float (&u0)[P], const float (&u1)[P]) {
-        using TR = typename std::remove_pointer<decltype(row)>::type;
-        if constexpr (!INTERLEAVED) {
-            store_f32<TR, P, true>(row + a0, u0);
-            store_f32<TR, P, true>(row + a1, u1);
-        } else {
-            float o[2 * P];
-#pragma unroll
-            for (int j = 0; j < P; ++j) {
-                o[2 * j] = u0[j];
-                o[2 * j + 1] = u1[j];
-            }
-            store_f32<TR, 2 * P, true>(row + a0, o);
+    float cs[P], sn[P];
+    if (eval) {
+        if (tid < 24) inv_pio4[tid] = tab_word;
+        __syncthreads();
+        if (has_angle) {
+            const float freq = ((float)apos / a.pos_scale) / den;
+            glibc_sincosf_tab(freq, inv_pio4, &sn_s[tk * a.half + pair], &cs_s[tk * a.half + pair]);
         }
-    };
-    for (int hh = h_begin; hh < h_end; ++hh) {
-        const bool is_q = hh < nq;
-        if (hh != h_begin) SPH_LOAD_HEAD(hh);
-        if (!is_q && !pos_ok) continue;
-        float o0[P], o1[P];
+        if constexpr (!kOwn) __syncthreads();
+        if (!active) return;
+        if constexpr (kOwn) glibc_sincosf_tab(((float)ps / a.pos_scale) / den, inv_pio4, &sn[0], &cs[0]);
+#pragma unroll
+        for (int j = 0; j < (kOwn ? 0 : P); ++j) {
+            cs[j] = cs_s[tl * a.half + i0 + j];
+            sn[j] = sn_s[tl * a.half + i0 + j];
+        }
+    } else {
+        // Angles supplied as (cos, sin) per (token, pair), or per position in a
+        // table of max_seq rows. A position outside the table reads no row: q is
+        // rotated by angle 0 (cos 1, sin 0), the caches are left alone and the flag set.
+        if (!active) return;
+        const bool in_table = !a.ang_by_pos || (ps >= 0 && (int64_t)ps < a.max_seq);
+        const int64_t row = a.ang_by_pos ? (in_table ? ps : 0) : s;
+        const float* ag = a.ang + 2 * ((size_t)row * (size_t)a.half + (size_t)i0);
 #pragma unroll
         for (int j = 0; j < P; ++j) {
-            o0[j] = x0[j] * cs[j] - x1[j] * sn[j];
-            o1[j] = x1[j] * cs[j] + x0[j] * sn[j];
+            cs[j] = in_table ? ag[2 * j] : 1.0f;
+            sn[j] = in_table ? ag[2 * j + 1] : 0.0f;
         }
-        if (is_q) {
-            put(qo + ((size_t)hh * (size_t)seq + (size_t)s) * (size_t)head_dim, o0, o1);
-        } else {
-            const size_t crow = ((size_t)(hh - nq) * (size_t)max_seq + (size_t)ps) * (size_t)head_dim;
+    }
+    const bool pos_ok = ps >= 0 && (int64_t)ps < a.max_seq;
+    if (!pos_ok && a.bad != nullptr && lit == 0) *a.bad = 1;
+
+    // Row values with the bias of their channels added (y + b in f32, then
+    // stored in the activation type before RoPE reads it: round through T).
+    auto values = [&](const Runs& raw, int which, const float (&b)[2 * P], float (&f)[2 * P]) {
+        raw.to_f32(f);
+        if (BIAS && a.bias[which] != nullptr) {
+#pragma unroll
+            for (int j = 0; j < 2 * P; ++j) f[j] = widen(narrow<T>(f[j] + b[j]));
+        }
+    };
+    auto rotate = [&](float (&f)[2 * P]) {
+#pragma unroll
+        for (int j = 0; j < P; ++j) {
+            const int A = INTERLEAVED ? 2 * j : j, B = INTERLEAVED ? 2 * j + 1 : P + j;
+            const float xa = f[A], xb = f[B];
+            f[A] = xa * cs[j] - xb * sn[j];
+            f[B] = xb * cs[j] + xa * sn[j];
+        }
+    };
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int h = h0 + u * a.heads;
+        if (h >= H) return;
+        float f[2 * P];
+        if (h < a.nq) {
+            values(x[u], 0, xb[BIAS ? u : 0], f);
+            rotate(f);
+            Runs::store(a.qo + ((size_t)h * (size_t)a.seq + (size_t)s) * (size_t)a.head_dim, i0, a.half, f);
+        } else if (pos_ok) {
+            const int hk = h - a.nq;
+            const size_t crow = ((size_t)hk * (size_t)a.max_seq + (size_t)ps) * (size_t)a.head_dim;
+            values(x[u], 1, xb[BIAS ? u : 0], f);
+            rotate(f);
             // The unfused sequence stores rotated k in the activation type
             // before converting it to the cache type: round through T first.
             if constexpr (!std::is_same<T, float>::value) {
 #pragma unroll
-                for (int j = 0; j < P; ++j) {
-                    o0[j] = widen(narrow<T>(o0[j]));
-                    o1[j] = widen(narrow<T>(o1[j]));
-                }
+                for (int j = 0; j < 2 * P; ++j) f[j] = widen(narrow<T>(f[j]));
             }
-            put(kc + crow, o0, o1);
-            put(vc + crow, v0, v1);  // v: the same channels, moved unrotated
+            Runs::store(a.kc + crow, i0, a.half, f);
+            values(w[u], 2, wb[BIAS ? u : 0], f);
+            Runs::store(a.vc + crow, i0, a.half, f);  // v: the same channels, moved unrotated
         }
     }
-#undef SPH_LOAD_HEAD
 }
 
 // Launch shape of rope_kernel per storage type and layout, chosen by
@@ -589,81 +640,98 @@ inline void fill_dens(DenTable& den, int half, int rotary_dim, float base) {
         den.v[i] = i < half ? powf(base, 2.0f * (float)i / (float)rotary_dim) : 1.0f;
 }
 
-template <typename T, typename TC, typename TB, int P, bool IL, bool TM>
-int launch_rope_kv_p(const T* q, T* qo, int nq, const T* k, const T* v, int nkv, const int32_t* pos, int64_t seq, int head_dim,
-                     float pos_scale, TC* kc, TC* vc, int64_t max_seq, int32_t* flag, const TB* bq, const TB* bk,
-                     const TB* bv, const DenTable& den, const float* ang, bool ang_by_pos, hipStream_t stream) {
-    const int half = head_dim / 2;
-    const int lanes_per_tok = half / P;
-    const int toks_per_block = kThreads / lanes_per_tok;
-    const int64_t blocks_x = (seq + toks_per_block - 1) / toks_per_block;
-    const int heads = nq + nkv;
-    // Blocks to aim for (head groups × token blocks), swept at the Llama-3-8B
-    // shape: f32 512; half types 512 NEOX, 1536 interleaved.
-    const int target = sizeof(T) == 4 ? 512 : (IL ? 1536 : 512);
-    int groups = (int)((target + blocks_x - 1) / blocks_x);
-    if (groups > heads) groups = heads;
-    if (groups < 1) groups = 1;
-    const int heads_per_group = (heads + groups - 1) / groups;
-    groups = (heads + heads_per_group - 1) / heads_per_group;
+// Launch shape, from the lanes that the rows need (one row per thread and pass):
+//  - small (up to 2^14: decode steps): blocks of one wave, so that the rows spread over the CUs, each with the
+//    angles of one token (two heads a block 2.96 us, four 3.14, one 3.00 at one token of 14 + 2 heads x 64);
+//  - up to 2^18: at most 64 angles a block, so that only some waves evaluate them, and from 2^16 on two rows
+//    per thread (512 tokens of 14 + 2 x 64 f32 4.1 us with 256 angles, 3.8 with 64; 333 of 32 + 8 x 128 bf16
+//    4.4 with one row, 4.0 with two; 64 tokens of 64 heads x 80 f16 4.4 with one, 4.8 with two);
+//  - larger: 256 angles, two rows (2048 tokens of 32 + 8 x 128 f16 10.9 us, with 64 angles 11.6).
+template <typename T, typename TC, int P, bool IL, bool TM>
+int launch_rope_kv_p(RopeKvArgs<T, TC>& a, hipStream_t stream) {
+    const int heads = a.nq + a.nkv;
+    a.lanes = a.half / P;
+    const int64_t lanes = a.seq * heads * a.lanes;
+    const bool small = lanes <= 1 << 14 && a.half <= 64;
+    const int threads = small ? kWave : kThreads;
+    const int rows = threads / a.lanes;  // of a block per pass: toks x heads
+    a.toks = (lanes < 1 << 18 ? 64 : kMaxBlockAngles) / a.half;
+    if (a.toks < 1) a.toks = 1;
+    if (a.toks > rows) a.toks = rows;
+    if (a.toks > a.seq) a.toks = (int)a.seq;
+    a.heads = rows / a.toks;
+    if (small && a.heads > 2) a.heads = 2;
+    if (a.heads > heads) a.heads = heads;
+    const int64_t blocks_x = (a.seq + a.toks - 1) / a.toks;
     if (blocks_x > INT32_MAX) return SPH_EINVAL;
-    const dim3 grid((unsigned)blocks_x, (unsigned)groups);
-    return launch(rope_kv_kernel<T, TC, TB, P, IL, TM>, grid, kThreads, stream, q, qo, nq, k, v, nkv, pos, seq,
-                  head_dim, half, lanes_per_tok, toks_per_block, heads_per_group, pos_scale, kc, vc, max_seq, flag, bq,
-                  bk, bv, den, ang, ang_by_pos);
+    const bool two = lanes >= 1 << 16;
+    const bool bias = a.bias[0] != nullptr || a.bias[1] != nullptr || a.bias[2] != nullptr;
+    const int tile = (two ? 2 : 1) * a.heads;  // heads per block
+    // Large launches pass the caches by: 8192 tokens of 32 + 8 x 128 f16 39.7 us cached, 35.1 non-temporal, but
+    // 333 tokens bf16 4.0 against 4.4 (kCachedBytes).
+    const int64_t row = (int64_t)a.head_dim * (TM ? 2 : 1) * (int64_t)sizeof(T);
+    const bool nt = two && a.seq * (a.nq * row + 2 * a.nkv * (int64_t)a.head_dim * (int64_t)(sizeof(T) + sizeof(TC))) >=
+                               kCachedBytes;
+    constexpr int64_t kMaxY = 65535;
+    for (int64_t h0 = 0; h0 < heads; h0 += kMaxY * tile) {
+        a.h_first = (int)h0;
+        const int64_t tiles = (heads - h0 + tile - 1) / tile;
+        const dim3 grid((unsigned)blocks_x, (unsigned)(tiles < kMaxY ? tiles : kMaxY));
+        auto go = [&](auto u, auto b, auto n) {
+            return launch(rope_kv_kernel<T, TC, P, IL, TM, decltype(u)::value, decltype(b)::value, decltype(n)::value>,
+                          grid, threads, stream, a);
+        };
+        using std::false_type;
+        using std::true_type;
+        const std::integral_constant<int, 1> one;
+        const std::integral_constant<int, 2> pair;
+        const int st = !two ? (bias ? go(one, true_type{}, false_type{}) : go(one, false_type{}, false_type{}))
+                       : nt ? (bias ? go(pair, true_type{}, true_type{}) : go(pair, false_type{}, true_type{}))
+                            : (bias ? go(pair, true_type{}, false_type{}) : go(pair, false_type{}, false_type{}));
+        if (st != SPH_OK) return st;
+    }
+    return SPH_OK;
 }
 
 // P: pairs per thread, the widest whose accesses of q/k/v (type T) and of the
 // caches (type TC) stay within 16 bytes and aligned.
-template <typename T, typename TC, typename TB, bool TM>
-int launch_rope_kv(const void* qv, void* qov, int nq, const void* kv, const void* vv, int nkv, int layout,
-                   const int32_t* pos, int64_t seq, int head_dim, float base, float pos_scale, void* kcv, void* vcv,
-                   int64_t max_seq, int32_t* flag, const void* bqv, const void* bkv, const void* bvv, const float* ang,
-                   bool ang_by_pos, hipStream_t stream) {
-    const TB* bq = static_cast<const TB*>(bqv);
-    const TB* bk = static_cast<const TB*>(bkv);
-    const TB* bv = static_cast<const TB*>(bvv);
-    const T* q = static_cast<const T*>(qv);
-    T* qo = static_cast<T*>(qov);
-    const T* k = static_cast<const T*>(kv);
-    const T* v = static_cast<const T*>(vv);
-    TC* kc = static_cast<TC*>(kcv);
-    TC* vc = static_cast<TC*>(vcv);
-    const int half = head_dim / 2;
+template <typename T, typename TC, bool TM>
+int launch_rope_kv(RopeKvArgs<T, TC>& a, int layout, float base, hipStream_t stream) {
+    a.half = a.head_dim / 2;
     // Supplied angles leave the denominators unused: no libm calls per launch.
-    DenTable den{};
-    if (ang == nullptr) fill_dens(den, half, head_dim, base);
+    if (a.ang == nullptr) fill_dens(a.den, a.half, a.head_dim, base);
     const bool il = layout == SPH_ROPE_INTERLEAVED;
+    const size_t sb = dtype_size(a.bias_dt);
     auto ok = [&](int P) {
         const int run = il ? 2 * P : P;  // contiguous elements per access
-        if (half % P != 0 || head_dim % run != 0) return false;
+        if (a.half % P != 0 || a.head_dim % run != 0) return false;
         if (run * sizeof(T) > 16 || run * sizeof(TC) > 16) return false;
         if ((run * sizeof(T)) % 4 != 0 || (run * sizeof(TC)) % 4 != 0) return false;
         const size_t at = run * sizeof(T) < 16 ? run * sizeof(T) : 16;
         const size_t ac = run * sizeof(TC) < 16 ? run * sizeof(TC) : 16;
-        const size_t ab = run * sizeof(TB) < 16 ? run * sizeof(TB) : 16;  // bias runs may span two 16-byte loads
-        return aligned(q, at) && aligned(qo, at) && aligned(k, at) && aligned(v, at) && aligned(kc, ac) &&
-               aligned(vc, ac) && aligned(bq, ab) && aligned(bk, ab) && aligned(bv, ab);
+        const size_t ab = run * sb < 16 ? run * sb : 16;  // bias runs may span two 16-byte loads
+        return aligned(a.q, at) && aligned(a.qo, at) && aligned(a.k, at) && aligned(a.v, at) && aligned(a.kc, ac) &&
+               aligned(a.vc, ac) && aligned(a.bias[0], ab) && aligned(a.bias[1], ab) && aligned(a.bias[2], ab);
     };
     constexpr int V = vec16<T>::n < vec16<TC>::n ? vec16<T>::n : vec16<TC>::n;
     // A decode step (a few tokens) leaves most lanes of its blocks idle and its
     // time is one dependent chain — position load, the thread's sin/cos, store —
-    // so it takes the narrowest runs that stay word-sized: fewer angles per lane.
-    const bool few = seq <= 4;
+    // so it takes the narrowest runs that stay word-sized.
+    const bool few = a.seq <= 4;
     if (!il) {
-        if (few && ok(V / 2)) return launch_rope_kv_p<T, TC, TB, V / 2, false, TM>(q, qo, nq, k, v, nkv, pos, seq, head_dim, pos_scale, kc, vc, max_seq, flag, bq, bk, bv, den, ang, ang_by_pos, stream);
-        if (ok(V)) return launch_rope_kv_p<T, TC, TB, V, false, TM>(q, qo, nq, k, v, nkv, pos, seq, head_dim, pos_scale, kc, vc, max_seq, flag, bq, bk, bv, den, ang, ang_by_pos, stream);
-        if (ok(V / 2)) return launch_rope_kv_p<T, TC, TB, V / 2, false, TM>(q, qo, nq, k, v, nkv, pos, seq, head_dim, pos_scale, kc, vc, max_seq, flag, bq, bk, bv, den, ang, ang_by_pos, stream);
+        if (few && ok(V / 2)) return launch_rope_kv_p<T, TC, V / 2, false, TM>(a, stream);
+        if (ok(V)) return launch_rope_kv_p<T, TC, V, false, TM>(a, stream);
+        if (ok(V / 2)) return launch_rope_kv_p<T, TC, V / 2, false, TM>(a, stream);
         if constexpr (V / 4 >= 2) {
-            if (ok(V / 4)) return launch_rope_kv_p<T, TC, TB, V / 4, false, TM>(q, qo, nq, k, v, nkv, pos, seq, head_dim, pos_scale, kc, vc, max_seq, flag, bq, bk, bv, den, ang, ang_by_pos, stream);
+            if (ok(V / 4)) return launch_rope_kv_p<T, TC, V / 4, false, TM>(a, stream);
         }
     } else {
         if constexpr (V / 4 >= 1) {
-            if (few && ok(V / 4)) return launch_rope_kv_p<T, TC, TB, V / 4, true, TM>(q, qo, nq, k, v, nkv, pos, seq, head_dim, pos_scale, kc, vc, max_seq, flag, bq, bk, bv, den, ang, ang_by_pos, stream);
+            if (few && ok(V / 4)) return launch_rope_kv_p<T, TC, V / 4, true, TM>(a, stream);
         }
-        if (ok(V / 2)) return launch_rope_kv_p<T, TC, TB, V / 2, true, TM>(q, qo, nq, k, v, nkv, pos, seq, head_dim, pos_scale, kc, vc, max_seq, flag, bq, bk, bv, den, ang, ang_by_pos, stream);
+        if (ok(V / 2)) return launch_rope_kv_p<T, TC, V / 2, true, TM>(a, stream);
         if constexpr (V / 4 >= 1) {
-            if (ok(V / 4)) return launch_rope_kv_p<T, TC, TB, V / 4, true, TM>(q, qo, nq, k, v, nkv, pos, seq, head_dim, pos_scale, kc, vc, max_seq, flag, bq, bk, bv, den, ang, ang_by_pos, stream);
+            if (ok(V / 4)) return launch_rope_kv_p<T, TC, V / 4, true, TM>(a, stream);
         }
     }
     return SPH_EINVAL;  // head_dim or alignment the vector paths do not cover
@@ -847,13 +915,28 @@ int rope_kv_entry(const void* q, void* q_out, int64_t n_q_heads, const void* k, 
         using T = decltype(t);
         return with_float_type(cache_dtype, [&](auto tc) -> int {
             using TC = decltype(tc);
-            return with_float_type(bias_dtype, [&](auto tb) -> int {
-                using TB = decltype(tb);
-                return launch_rope_kv<T, TC, TB, TM>(q, q_out, (int)n_q_heads, k, v, (int)n_kv_heads, layout,
-                                                     positions, seq, (int)head_dim, base, pos_scale, kcache, vcache,
-                                                     max_seq, bad_pos_flag, bq, bk, bv, angles,
-                                                     angles_by_position, s);
-            });
+            RopeKvArgs<T, TC> a{};
+            a.q = static_cast<const T*>(q);
+            a.qo = static_cast<T*>(q_out);
+            a.k = static_cast<const T*>(k);
+            a.v = static_cast<const T*>(v);
+            a.kc = static_cast<TC*>(kcache);
+            a.vc = static_cast<TC*>(vcache);
+            a.pos = positions;
+            a.bias[0] = bq;
+            a.bias[1] = bk;
+            a.bias[2] = bv;
+            a.bias_dt = bias_dtype;
+            a.nq = (int)n_q_heads;
+            a.nkv = (int)n_kv_heads;
+            a.seq = seq;
+            a.max_seq = max_seq;
+            a.head_dim = (int)head_dim;
+            a.pos_scale = pos_scale;
+            a.bad = bad_pos_flag;
+            a.ang = angles;
+            a.ang_by_pos = angles_by_position;
+            return launch_rope_kv<T, TC, TM>(a, layout, base, s);
         });
     });
 }

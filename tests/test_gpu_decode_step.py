@@ -233,3 +233,55 @@ def test_token_major_variant_rejects_overlap_and_flags_bad_positions(dev):
     nz = (kc.abs().sum(dim=(0, 2)) > 0).cpu().tolist()
     assert nz == [False, False, True, False, False, False, False, False]
     assert (vc.abs().sum(dim=(0, 2)) > 0).cpu().tolist() == nz
+
+
+# Fused against unfused (add_bias, transpose, rope, kv_append: each checked against the oracle elsewhere), bit for
+# bit, around the launch shapes' bounds: one wave per block up to 2^14 lanes, two rows per thread from 2^16, 256
+# angles a block from 2^18, non-temporal from 2^27 bytes; head dims whose pairs do not divide a block (80, 96),
+# the largest (512), pairs one by one (interleaved, a few tokens), some of the biases absent.
+@pytest.mark.parametrize("dtype,kv,T,nq,nkv,hd,il,bias", [
+    (torch.float32, torch.float16, 1, 14, 2, 64, False, "qkv"), (torch.float32, torch.float16, 3, 14, 2, 64, True, "qkv"),
+    (torch.float32, torch.float32, 4, 5, 5, 80, True, "k"), (torch.float16, torch.float16, 5, 7, 1, 96, False, "v"),
+    (torch.bfloat16, torch.bfloat16, 127, 16, 0, 128, False, ""), (torch.bfloat16, torch.bfloat16, 129, 0, 16, 64, True, "k"),
+    (torch.float32, torch.bfloat16, 511, 14, 2, 64, False, "q"), (torch.float32, torch.bfloat16, 513, 14, 2, 64, False, "qkv"),
+    (torch.float16, torch.float16, 333, 32, 8, 128, True, ""), (torch.float16, torch.float32, 100, 4, 4, 512, False, "qv"),
+    (torch.float16, torch.float16, 1031, 32, 8, 128, False, "qkv"), (torch.bfloat16, torch.bfloat16, 820, 40, 40, 80, True, "qk"),
+    (torch.float32, torch.float16, 3001, 32, 8, 128, True, "qkv"), (torch.float16, torch.float16, 7001, 32, 8, 128, False, "")])
+@pytest.mark.parametrize("tokens", [False, True], ids=["heads", "tokens"])
+def test_fused_step_launch_shapes(dev, dtype, kv, T, nq, nkv, hd, il, bias, tokens):
+    print(f"case fused shapes {dtype} {kv} T {T} heads {nq}+{nkv}x{hd} il {il} bias '{bias}' tokens {tokens}", flush=True)
+    g = torch.Generator(device=dev).manual_seed(T * 7 + hd)
+    rnd = lambda *s: torch.randn(s, generator=g, device=dev)
+    q, k, v = rnd(nq, T, hd).to(dtype), rnd(nkv, T, hd).to(dtype), rnd(nkv, T, hd).to(dtype)
+    b = {n: rnd(h * hd) for n, h in zip("qkv", (nq, nkv, nkv)) if n in bias and h}
+    max_seq, start = T + 70, 41
+    pos = torch.arange(start, start + T, dtype=torch.int32, device=dev)
+    caches = [torch.zeros(nkv, max_seq, hd, dtype=kv, device=dev) for _ in range(4)]
+
+    def biased(x, n):
+        if n not in b:
+            return x.clone()
+        t = x.transpose(0, 1).contiguous()
+        return ops.add_bias(t.view(T, -1), b[n]).view(t.shape).transpose(0, 1).contiguous()
+
+    wq, wk, wv = biased(q, "q"), biased(k, "k"), biased(v, "v")
+    if nq:
+        ops.rope_(wq[None], None, pos, 1e4, interleaved=il)
+    if nkv:
+        ops.rope_(wk[None], None, pos, 1e4, interleaved=il)
+        ops.kv_append(wk, caches[0], start)
+        ops.kv_append(wv, caches[1], start)
+    args = dict(interleaved=il, bq=b.get("q"), bk=b.get("k"), bv=b.get("v"))
+    if tokens:
+        tm = lambda x: x.transpose(0, 1).contiguous()
+        got = ops.rope_kv_append_tokens(tm(q), tm(k), tm(v), pos, 1e4, caches[2], caches[3], **args)
+    else:
+        got = q.clone()
+        ops.rope_kv_append(got, k, v, pos, 1e4, caches[2], caches[3], **args)
+    torch.cuda.synchronize()
+    same = lambda x, y: torch.equal(x.contiguous().view(torch.uint8), y.contiguous().view(torch.uint8))
+    if nq:
+        assert same(got, wq), "q"
+    if nkv:
+        assert same(caches[2], caches[0]), "k cache"
+        assert same(caches[3], caches[1]), "v cache"
