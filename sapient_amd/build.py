@@ -4,7 +4,9 @@ Each ``csrc/*.hip`` / ``csrc/*.cpp`` kernel translation unit and the C++
 host layer (``host/*.cpp``) is compiled by hipcc (in parallel) into
 ``sapient_amd/_build/`` and linked into one shared library that exports the C
 ABI declared in ``include/sapient_hip.h`` and the C++ API of
-``include/sapient_hip_backend.hpp``.
+``include/sapient_hip_backend.hpp``. The native half of :mod:`sapient_amd.ops`
+(``binding/torch_ops.cpp``, against torch's headers) is compiled by g++ into
+``sapient_amd/_torch_ops.so``, which links that library.
 
 Usage: ``python -m sapient_amd.build`` (or ``__graft_entry__.build()``).
 """
@@ -22,6 +24,7 @@ ROOT = PKG.parent
 CSRC = PKG / "csrc"
 BUILD = PKG / "_build"
 LIB = PKG / "libsapient_hip.so"
+BINDING = PKG / "_torch_ops.so"
 
 ARCH = "gfx950"
 
@@ -70,6 +73,25 @@ def _compile(src: Path) -> Path:
     return obj
 
 
+def _build_binding() -> None:
+    """The torch binding: host code only, in torch's own C++ ABI, found beside the library at run time."""
+    import sysconfig
+
+    import torch
+    t = Path(torch.__file__).parent
+    tmp = BINDING.with_suffix(".so.tmp")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}", f"-I{ROOT / 'include'}",
+           "-isystem", str(t / "include"), "-isystem", str(t / "include" / "torch" / "csrc" / "api" / "include"),
+           "-isystem", "/opt/rocm/include", "-isystem", sysconfig.get_paths()["include"],
+           str(PKG / "binding" / "torch_ops.cpp"), "-o", str(tmp), f"-L{PKG}", f"-l:{LIB.name}", f"-L{t / 'lib'}",
+           "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed for torch_ops.cpp:\n{res.stderr}")
+    os.replace(tmp, BINDING)
+
+
 def build(verbose: bool = True) -> Path:
     """Compile every translation unit for gfx950 and link the shared library."""
     BUILD.mkdir(exist_ok=True)
@@ -84,6 +106,7 @@ def build(verbose: bool = True) -> Path:
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stderr}")
     os.replace(tmp, LIB)
+    _build_binding()
     if verbose:
         print(f"built {LIB.relative_to(ROOT)} from {len(srcs)} sources")
     return LIB

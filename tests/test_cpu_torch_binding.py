@@ -1,0 +1,31 @@
+"""The native op calls (binding/torch_ops.cpp) without a GPU: every function of ops.py reaches its argument
+checks with the arguments it documents, and refuses what is not a contiguous device tensor."""
+import pytest
+import torch
+
+import sapient_amd.ops as ops
+
+X, I = torch.zeros(1, 2, 3, 4), torch.zeros(3, dtype=torch.int32)
+CALLS = {
+    "rms_norm": lambda t: ops.rms_norm(t, None, 1e-5, out_dtype=torch.float32),
+    "layer_norm": lambda t: ops.layer_norm(t, None, None, 1e-5),
+    "add_rms_norm": lambda t: ops.add_rms_norm(t, t, None, 1e-5, sum_out=t),
+    "add": lambda t: ops.add(t, t), "mul": lambda t: ops.mul(t, t, out=t), "silu": ops.silu,
+    "swiglu": lambda t: ops.swiglu(t, t), "gelu_tanh": ops.gelu_tanh, "gelu_erf": lambda t: ops.gelu_erf(t, out=t),
+    "add_bias": lambda t: ops.add_bias(t, t),
+    "rope_": lambda t: ops.rope_(t, None, I, 1e4, rotary_dim=2, interleaved=True),
+    "rope_cached_": lambda t: ops.rope_cached_(t, t, t, t, positions=I, bad_pos_flag=I),
+    "embed": lambda t: ops.embed(t, 0, 3, 4, I, bad_id_flag=I), "transpose_heads": lambda t: ops.transpose_heads(t),
+    "kv_append": lambda t: ops.kv_append(t, t, 0), "kv_cache_update": lambda t: ops.kv_cache_update(t, t, 0),
+    "kv_cache_update_into": lambda t: ops.kv_cache_update_into(t, t, t, 0),
+    "rope_kv_append": lambda t: ops.rope_kv_append(t, t, t, I, 1e4, t, t, bq=t),
+    "rope_kv_append_tokens": lambda t: ops.rope_kv_append_tokens(t, t, t, I, 1e4, t, t, bv=t, out=t),
+}
+
+
+@pytest.mark.parametrize("name", CALLS)
+def test_refuses_host_tensors_and_other_objects(name):
+    with pytest.raises(ValueError, match="must be a device tensor"):
+        CALLS[name](X)
+    with pytest.raises(TypeError, match="must be a torch.Tensor"):
+        CALLS[name](object())
