@@ -268,13 +268,13 @@ __global__ __launch_bounds__(W >= 4 ? 64 * W : 256) void rms_rows_ragged(const T
     const size_t base = (size_t)(live ? row : 0) * (size_t)dim;
     const int e0 = ((wv % W) * VPT * kWave + lane) * E;  // this lane's first element; its runs lie kWave * E apart
 
-    u32x4 cx[VPT], cres[VPT];
+    uint32_t cx[VPT][4], cres[VPT][4];
 #pragma unroll
     for (int j = 0; j < VPT; ++j) {
         const int i = e0 + j * kWave * E;
         if (live && i < dim) {
-            cx[j] = load_run16<TX, NT>(x + base + i, dim - i);
-            if constexpr (adds(KIND)) cres[j] = load_run16<TX, NT>(residual + base + i, dim - i);
+            load_run<TX, E, NT>(x + base + i, dim - i, cx[j]);
+            if constexpr (adds(KIND)) load_run<TX, E, NT>(residual + base + i, dim - i, cres[j]);
         }
     }
     float r[VPT][E];
@@ -283,10 +283,10 @@ __global__ __launch_bounds__(W >= 4 ? 64 * W : 256) void rms_rows_ragged(const T
     for (int j = 0; j < VPT; ++j) {
         const int i = e0 + j * kWave * E;
         if (live && i < dim) {
-            unpack16<TX, E>(cx[j], r[j]);  // elements past the row's end are 0 and add nothing
+            words_to_f32<TX, E>(cx[j], r[j]);  // elements past the row's end are 0 and add nothing
             if constexpr (adds(KIND)) {
                 float b[E];
-                unpack16<TX, E>(cres[j], b);
+                words_to_f32<TX, E>(cres[j], b);
 #pragma unroll
                 for (int e = 0; e < E; ++e) r[j][e] = r[j][e] + b[e];
                 store_run_f32<TX, E, NT>((KIND == K_ADD_RMS_TO ? sum : residual) + base + i, dim - i, r[j]);

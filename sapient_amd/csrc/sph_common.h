@@ -173,62 +173,75 @@ __device__ __forceinline__ void store_f32(T* __restrict__ p, const float (&v)[N]
 // lane; only the cache lines that a wave's 1 KiB straddles are requested twice.
 typedef u32x4 u32x4_at4 __attribute__((aligned(4)));
 typedef u32x4 u32x4_at2 __attribute__((aligned(2)));
-template <typename T> struct elem_vec16 { typedef u32x4_at2 type; };
-template <> struct elem_vec16<float> { typedef u32x4_at4 type; };
+typedef u32x2 u32x2_at4 __attribute__((aligned(4)));
+typedef u32x2 u32x2_at2 __attribute__((aligned(2)));
+template <typename T, int BYTES> struct elem_vec;
+template <> struct elem_vec<float, 16> { typedef u32x4_at4 type; };
+template <> struct elem_vec<f16, 16> { typedef u32x4_at2 type; };
+template <> struct elem_vec<bf16, 16> { typedef u32x4_at2 type; };
+template <> struct elem_vec<float, 8> { typedef u32x2_at4 type; };
+template <> struct elem_vec<f16, 8> { typedef u32x2_at2 type; };
+template <> struct elem_vec<bf16, 8> { typedef u32x2_at2 type; };
 
-// The first min(n, E) of E consecutive elements (16 bytes of T) as raw words; the rest read as zero bits.
-template <typename T, bool NT>
-__device__ __forceinline__ u32x4 load_run16(const T* p, int n) {
-    constexpr int E = vec16<T>::n;
-    if (n >= E) {
-        // Not vload / vstore: a template parameter deduced from the pointer would drop its alignment.
-        const auto* a = reinterpret_cast<const typename elem_vec16<T>::type*>(p);
-        if constexpr (NT) return __builtin_nontemporal_load(a);
-        else return *a;
-    }
-    u32x4 q = {0u, 0u, 0u, 0u};
-#pragma unroll
-    for (int e = 0; e < E; ++e) {
-        if (e < n) {
-            if constexpr (sizeof(T) == 4) q[e] = __builtin_bit_cast(uint32_t, p[e]);
-            else q[e / 2] |= (uint32_t)__builtin_bit_cast(uint16_t, p[e]) << (16 * (e & 1));
-        }
-    }
-    return q;
-}
-
-// The first min(n, N) of N consecutive elements as f32 (N a multiple of T's 16-byte run).
+// The first min(n, N) of N consecutive elements as raw words, the rest zero bits; in accesses of
+// 16 bytes (8 where N elements are 8 bytes).
 template <typename T, int N, bool NT>
-__device__ __forceinline__ void load_run_f32(const T* p, int n, float (&v)[N]) {
-    constexpr int E = vec16<T>::n;
-    uint32_t raw[words_of<T, N>::n];
+__device__ __forceinline__ void load_run(const T* p, int n, uint32_t (&raw)[words_of<T, N>::n]) {
+    constexpr int B = N * (int)sizeof(T) >= 16 ? 16 : 8, E = B / (int)sizeof(T), W = B / 4;
+    static_assert(N % E == 0, "whole accesses");
 #pragma unroll
     for (int c = 0; c < N / E; ++c) {
-        const u32x4 q = load_run16<T, NT>(p + c * E, n - c * E);
-        raw[4 * c] = q.x; raw[4 * c + 1] = q.y; raw[4 * c + 2] = q.z; raw[4 * c + 3] = q.w;
+        if (n >= (c + 1) * E) {
+            // Not vload / vstore: a template parameter deduced from the pointer would drop its alignment.
+            const auto* a = reinterpret_cast<const typename elem_vec<T, B>::type*>(p + c * E);
+            typename elem_vec<T, B>::type q;
+            if constexpr (NT) q = __builtin_nontemporal_load(a);
+            else q = *a;
+#pragma unroll
+            for (int w = 0; w < W; ++w) raw[c * W + w] = q[w];
+        } else {
+#pragma unroll
+            for (int w = 0; w < W; ++w) raw[c * W + w] = 0u;
+#pragma unroll
+            for (int e = 0; e < E; ++e) {
+                if (c * E + e < n) {
+                    if constexpr (sizeof(T) == 4) raw[c * W + e] = __builtin_bit_cast(uint32_t, p[c * E + e]);
+                    else raw[c * W + e / 2] |= (uint32_t)__builtin_bit_cast(uint16_t, p[c * E + e]) << (16 * (e & 1));
+                }
+            }
+        }
     }
+}
+
+// The same as f32.
+template <typename T, int N, bool NT>
+__device__ __forceinline__ void load_run_f32(const T* p, int n, float (&v)[N]) {
+    uint32_t raw[words_of<T, N>::n];
+    load_run<T, N, NT>(p, n, raw);
     words_to_f32<T, N>(raw, v);
 }
 
 // Store the first min(n, N) of N f32 values as consecutive elements of T.
 template <typename T, int N, bool NT>
 __device__ __forceinline__ void store_run_f32(T* p, int n, const float (&v)[N]) {
-    constexpr int E = vec16<T>::n;
+    constexpr int B = N * (int)sizeof(T) >= 16 ? 16 : 8, E = B / (int)sizeof(T), W = B / 4;
     uint32_t raw[words_of<T, N>::n];
     f32_to_words<T, N>(v, raw);
 #pragma unroll
     for (int c = 0; c < N / E; ++c) {
         if (n >= (c + 1) * E) {
-            const u32x4 q = {raw[4 * c], raw[4 * c + 1], raw[4 * c + 2], raw[4 * c + 3]};
-            auto* a = reinterpret_cast<typename elem_vec16<T>::type*>(p + c * E);
+            auto* a = reinterpret_cast<typename elem_vec<T, B>::type*>(p + c * E);
+            typename elem_vec<T, B>::type q;
+            if constexpr (W == 4) q = u32x4{raw[c * W], raw[c * W + 1], raw[c * W + 2], raw[c * W + 3]};
+            else q = u32x2{raw[c * W], raw[c * W + 1]};
             if constexpr (NT) __builtin_nontemporal_store(q, a);
             else *a = q;
         } else {
 #pragma unroll
             for (int e = 0; e < E; ++e) {
                 if (c * E + e < n) {
-                    if constexpr (sizeof(T) == 4) p[c * E + e] = __builtin_bit_cast(T, raw[4 * c + e]);
-                    else p[c * E + e] = __builtin_bit_cast(T, (uint16_t)(raw[4 * c + e / 2] >> (16 * (e & 1))));
+                    if constexpr (sizeof(T) == 4) p[c * E + e] = __builtin_bit_cast(T, raw[c * W + e]);
+                    else p[c * E + e] = __builtin_bit_cast(T, (uint16_t)(raw[c * W + e / 2] >> (16 * (e & 1))));
                 }
             }
         }

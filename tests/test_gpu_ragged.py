@@ -72,3 +72,47 @@ def test_ragged_norms(dev, orc, dtype, rows, dim, off):
         # No row is skipped: every row's RMS is 1 where the weight is 1.
         u = ops.rms_norm(x, None, 0.0, out_dtype=torch.float32)
         assert (u.square().mean(-1) - 1).abs().max().item() < 1e-4
+
+
+# Element-wise launches around every bound of their dispatch (2^18 .. 2^21 elements, 2^20 vectors, 16 and 128 MB of
+# traffic), a few elements past each (short last runs) and at odd addresses, against the same op over pieces of at
+# most 2^18 elements at aligned addresses: the one-element kernel, which the other tests check against the oracle.
+def _pieces(fn, *xs):
+    step = 1 << 18
+    n = max(x.numel() for x in xs)
+    cut = lambda x, i: x if x.numel() == 1 else x.reshape(-1)[i:i + step].clone()
+    return torch.cat([fn(*[cut(x, i) for x in xs]).reshape(-1) for i in range(0, n, step)])
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=DT_ID)
+@pytest.mark.parametrize("n", [1, 2049, (1 << 18) + 1, (1 << 19) - 3, (1 << 19) + 8, (1 << 20) + 5, (1 << 21) + 2,
+                               (1 << 22) + 4, (1 << 22) + 7, (1 << 23) + 1, 23_000_000])
+@pytest.mark.parametrize("off", [0, 1])
+def test_elementwise_launch_bounds(dev, dtype, n, off):
+    print(f"case elementwise {dtype} n {n} offset {off}", flush=True)
+    x, u = _gen((n,), 11, dev, dtype, off, 2.0), _gen((n,), 12, dev, dtype, off, 2.0)
+    one = _gen((1,), 13, dev, dtype)
+    same = lambda a, b, what: torch.equal(a.reshape(-1).view(torch.uint8), b.reshape(-1).view(torch.uint8)) or pytest.fail(what)
+    for name, fn in (("silu", ops.silu), ("gelu_tanh", ops.gelu_tanh), ("gelu_erf", ops.gelu_erf)):
+        same(fn(x), _pieces(fn, x), name)
+    for name, fn in (("swiglu", ops.swiglu), ("add", ops.add), ("mul", ops.mul)):
+        same(fn(x, u), _pieces(fn, x, u), name)
+    if n > 1:
+        same(ops.add(x, one), _pieces(ops.add, x, one), "add scalar")
+        same(ops.mul(one, x), _pieces(ops.mul, one, x), "scalar mul")
+    want = _pieces(ops.swiglu, x, u)
+    assert ops.swiglu(x, u, out=x) is x  # in place
+    same(x, want, "swiglu in place")
+
+
+@pytest.mark.parametrize("dtype", DTYPES, ids=DT_ID)
+@pytest.mark.parametrize("rows,n,off", [(3, 1, 0), (5, 7, 1), (1, 2049, 0), (1100, 1001, 0), (1100, 1001, 1), (1048, 1000, 1),
+                                        (2049, 2048, 3), (700, 4097, 0), (4000, 9001, 0)])
+def test_ragged_bias(dev, orc, dtype, rows, n, off):
+    print(f"case ragged bias {dtype} {rows}x{n} offset {off}", flush=True)
+    y = _gen((rows, n), 21, dev, dtype, off)
+    for bdt in {torch.float32, torch.float16, dtype}:
+        b = _gen((n,), 22, dev, bdt, off)
+        got = ops.add_bias(y, b)
+        # y + b in f32, rounded once
+        assert torch.equal(got.view(torch.uint8), (y.float() + b.float()).to(dtype).view(torch.uint8))
