@@ -377,26 +377,46 @@ __global__ __launch_bounds__(kThreads) void gelu_lut_build(int which) {
     gelu_lut[which][slot] = narrow<T>(g).bits;
 }
 
-constexpr int kLutThreads = 512;
-constexpr int kLutBatch = 2;  // 16-byte vectors per thread per trip
+constexpr int kLutOneThreads = 1024, kLutTwoThreads = 512;  // one and two blocks per CU
 
 template <typename T>
 __device__ __forceinline__ uint32_t gelu_lookup(const uint16_t* tab, uint32_t h) {
     return (h & 0x7FFFu) < gelu_band<T>::kLimit ? (uint32_t)tab[gelu_slot<T>(h)] : gelu_outside<T>(h);
 }
 
-// Two 512-thread blocks per CU, both resident (LDS-bound), each staging the
-// band table in LDS once and then streaming 16-byte vectors, grid-stride, U
-// per thread per trip. Measured on MI355X at [8192, 10240] f16, round-robin
-// with a 16-byte copy of the same bytes (53.9 µs in this loop shape, 53.1 as
-// a flat grid): U = 2 56.8 µs, U = 3 58.6, U = 4 59.4, U = 1 62.8; four
-// blocks per CU (the table staged twice per slot) 59.4 at U = 2; the first
-// trip's loads issued before the table is staged: no change. Earlier:
-// 1024-thread blocks or the next trip's loads issued ahead (software
-// pipelining) 63-65.
-template <typename T, int U>
-__global__ __launch_bounds__(kLutThreads) void gelu_lut_apply(const uint16_t* in, uint16_t* out, int64_t nvec, int which) {
+// Blocks of THREADS that each stage the band table in LDS once and then stream
+// 16-byte runs, grid-stride, U per thread per trip, at any element alignment (the
+// thread whose run crosses the end takes its elements one by one), past the
+// caches at every size: erf-GELU f16 after the bias that wrote its input, 1500 x
+// 5120, 7.5 µs against 8.8 with cached loads and 3000 x 5120 14.2 against 17.2.
+//  - Up to one trip of 1024 threads x 4 runs on every CU (8 M elements): one block
+//    per CU, so the table is staged once, the fewest U that make it one trip, and
+//    all of a thread's loads in flight beside the table's (AHEAD). In the same
+//    sequence 400 x 5120 4.19 -> 3.72 µs, 800 x 5120 5.51 -> 4.85, 1500 x 5120 9.13 ->
+//    7.54 (8.3 with the loads after the table, 9.1 with two blocks of 512).
+//  - Larger: two 512-thread blocks per CU, both resident (LDS-bound), U = 2. At
+//    [8192, 10240] f16, round-robin with a 16-byte copy of the same bytes (53.9 µs
+//    in this loop shape, 53.1 as a flat grid): U = 2 56.8 µs, U = 3 58.6, U = 4 59.4,
+//    U = 1 62.8; four blocks per CU (the table staged twice per slot) 59.4 at U = 2;
+//    the first trip's loads issued before the table is staged: no change;
+//    1024-thread blocks 58.5, the next trip's loads issued ahead 63-65.
+template <typename T, int THREADS, int U, bool AHEAD>
+__global__ __launch_bounds__(THREADS) void gelu_lut_apply(const T* in, T* out, int64_t n, int which) {
+    constexpr int E = vec16<T>::n;
     __shared__ __align__(16) uint16_t tab[kLutEntries];
+    const int64_t nrun = (n + E - 1) / E;
+    const int64_t stride = (int64_t)gridDim.x * THREADS * U;
+    const int64_t first = (int64_t)blockIdx.x * THREADS * U + threadIdx.x;
+    // Elements of run i.
+    auto left = [&](int64_t i) { return i == nrun - 1 ? (int)(n - i * E) : E; };
+    uint32_t q[U][4];
+    auto load = [&](int64_t base) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int64_t i = base + (int64_t)u * THREADS;
+            if (i < nrun) load_run<T, E, true>(in + i * E, left(i), q[u]);
+        }
+    };
     {
         // The table is copied into LDS with gfx950's direct-to-LDS 16-byte
         // loads (global_load_lds_dwordx4: lane l of a wave writes the 16 bytes
@@ -405,57 +425,50 @@ __global__ __launch_bounds__(kLutThreads) void gelu_lut_apply(const uint16_t* in
         // (a load-wait-store loop through registers serialised ten of them; the
         // register-staged form of the same loop measured 0.2-0.4 us slower).
         constexpr int nq = (int)(2 * gelu_band<T>::kLimit * 2 / 16);  // 16-byte chunks of this type's table
-        constexpr int per = (nq + kLutThreads - 1) / kLutThreads;
+        constexpr int per = (nq + THREADS - 1) / THREADS;
         // A wave loads 64 chunks from its base, and only waves whose base is below nq load.
         static_assert((nq + 63) / 64 * 64 <= (int)(kLutEntries * 2 / 16), "a wave's chunks stay inside tab");
         const u32x4* src = reinterpret_cast<const u32x4*>(gelu_lut[which]);
         const int wv = (int)threadIdx.x / 64;
 #pragma unroll
         for (int i = 0; i < per; ++i) {
-            const int base = i * kLutThreads + wv * 64;  // this wave's first chunk (wave-uniform)
+            const int base = i * THREADS + wv * 64;  // this wave's first chunk (wave-uniform)
             if (base < nq) {
                 // Lanes past the table's end reload its last chunk into tab's
                 // spare slots (in bounds: see the static_assert).
-                const int k = (int)threadIdx.x + i * kLutThreads;
+                const int k = (int)threadIdx.x + i * THREADS;
                 __builtin_amdgcn_global_load_lds(src + (k < nq ? k : nq - 1), reinterpret_cast<u32x4*>(tab) + base,
                                                  16, 0, 0);
             }
         }
+        if constexpr (AHEAD) load(first);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
     __syncthreads();
-    const u32x4* vin = reinterpret_cast<const u32x4*>(in);
-    u32x4* vout = reinterpret_cast<u32x4*>(out);
-    const int64_t stride = (int64_t)gridDim.x * kLutThreads * U;
-    for (int64_t base = (int64_t)blockIdx.x * kLutThreads * U + threadIdx.x; base < nvec; base += stride) {
-        u32x4 q[U];
+    for (int64_t base = first; base < nrun; base += stride) {
+        if (!AHEAD || base != first) load(base);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int64_t i = base + (int64_t)u * kLutThreads;
-            if (i < nvec) q[u] = vload<true>(vin + i);
-        }
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const int64_t i = base + (int64_t)u * kLutThreads;
-            if (i < nvec) {
-                u32x4 r;
+            const int64_t i = base + (int64_t)u * THREADS;
+            if (i < nrun) {
+                uint32_t r[4];
 #pragma unroll
                 for (int c = 0; c < 4; ++c) {
                     const uint32_t w = q[u][c];
                     r[c] = gelu_lookup<T>(tab, w & 0xFFFFu) | (gelu_lookup<T>(tab, w >> 16) << 16);
                 }
-                vstore<true>(vout + i, r);
+                store_run_words<T, E, true>(out + i * E, left(i), r);
             }
         }
     }
 }
 
+// One element per thread, the table read from cache (see kFewElems).
 template <typename T>
-__global__ __launch_bounds__(kThreads) void gelu_lut_apply_scalar(const uint16_t* in, uint16_t* out, int64_t begin,
-                                                                  int64_t end, int which) {
+__global__ __launch_bounds__(kThreads) void gelu_lut_apply_scalar(const T* in, T* out, int64_t n, int which) {
     const int64_t stride = (int64_t)gridDim.x * kThreads;
-    for (int64_t i = begin + (int64_t)blockIdx.x * kThreads + threadIdx.x; i < end; i += stride)
-        out[i] = (uint16_t)gelu_lookup<T>(gelu_lut[which], in[i]);
+    for (int64_t i = (int64_t)blockIdx.x * kThreads + threadIdx.x; i < n; i += stride)
+        out[i].bits = (uint16_t)gelu_lookup<T>(gelu_lut[which], in[i].bits);
 }
 
 constexpr int kMaxDevices = 64;
@@ -491,29 +504,26 @@ int ensure_device_ready(hipStream_t stream, int* cus) {
 }
 
 template <typename T>
-int gelu_half(const uint16_t* x, uint16_t* out, int which, int64_t n, hipStream_t stream) {
+int gelu_half(const void* x, void* out, int which, int64_t n, hipStream_t stream) {
     int cus = 0;
-    int st = ensure_device_ready(stream, &cus);
+    const int st = ensure_device_ready(stream, &cus);
     if (st != SPH_OK) return st;
-    if (n <= kFewElems)  // one element per thread, the table read from cache (see kFewElems)
-        return launch(gelu_lut_apply_scalar<T>, grid_for(n, kThreads, 4096), kThreads, stream, x, out, (int64_t)0, n,
-                      which);
-    int64_t done = 0;
-    if (aligned(x, 16) && aligned(out, 16)) {
-        const int64_t nvec = n / 8;
-        if (nvec > 0) {
-            st = launch(gelu_lut_apply<T, kLutBatch>, grid_for(nvec, (int64_t)kLutThreads * kLutBatch, 2 * cus),
-                        kLutThreads, stream, x, out, nvec, which);
-            if (st != SPH_OK) return st;
-        }
-        done = nvec * 8;
-    }
-    if (done < n) {
-        st = launch(gelu_lut_apply_scalar<T>, grid_for(n - done, kThreads, 4096), kThreads, stream, x, out, done, n,
-                    which);
-        if (st != SPH_OK) return st;
-    }
-    return SPH_OK;
+    const T* xp = static_cast<const T*>(x);
+    T* op = static_cast<T*>(out);
+    if (n <= kFewElems)
+        return launch(gelu_lut_apply_scalar<T>, grid_for(n, kThreads, 4096), kThreads, stream, xp, op, n, which);
+    const int64_t nrun = (n + vec16<T>::n - 1) / vec16<T>::n;
+    const int64_t trip = (int64_t)cus * kLutOneThreads;  // runs of one trip, one per thread
+    auto one = [&](auto u) {
+        constexpr int U = decltype(u)::value;
+        return launch(gelu_lut_apply<T, kLutOneThreads, U, true>, grid_for(nrun, (int64_t)kLutOneThreads * U, cus),
+                      kLutOneThreads, stream, xp, op, n, which);
+    };
+    if (nrun <= trip) return one(std::integral_constant<int, 1>{});
+    if (nrun <= 2 * trip) return one(std::integral_constant<int, 2>{});
+    if (nrun <= 4 * trip) return one(std::integral_constant<int, 4>{});
+    return launch(gelu_lut_apply<T, kLutTwoThreads, 2, false>, grid_for(nrun, kLutTwoThreads * 2, 2 * cus),
+                  kLutTwoThreads, stream, xp, op, n, which);
 }
 
 // GELU of either form: half types through the tables, f32 per element.
@@ -523,10 +533,8 @@ int gelu_any(const void* x, void* out, int dtype, int64_t n, hipStream_t s) {
     if (n > 0 && (x == nullptr || out == nullptr)) return SPH_EINVAL;
     if (n == 0) return is_float_dtype(dtype) ? SPH_OK : SPH_EINVAL;
     const int form = OP == OP_GELU ? 0 : 1;
-    if (dtype == SPH_F16)
-        return gelu_half<f16>(static_cast<const uint16_t*>(x), static_cast<uint16_t*>(out), form * 2, n, s);
-    if (dtype == SPH_BF16)
-        return gelu_half<bf16>(static_cast<const uint16_t*>(x), static_cast<uint16_t*>(out), form * 2 + 1, n, s);
+    if (dtype == SPH_F16) return gelu_half<f16>(x, out, form * 2, n, s);
+    if (dtype == SPH_BF16) return gelu_half<bf16>(x, out, form * 2 + 1, n, s);
     return dispatch_unary<OP>(x, out, dtype, n, s);
 }
 

@@ -221,12 +221,10 @@ __device__ __forceinline__ void load_run_f32(const T* p, int n, float (&v)[N]) {
     words_to_f32<T, N>(raw, v);
 }
 
-// Store the first min(n, N) of N f32 values as consecutive elements of T.
+// Store the first min(n, N) of N consecutive elements, held as raw words.
 template <typename T, int N, bool NT>
-__device__ __forceinline__ void store_run_f32(T* p, int n, const float (&v)[N]) {
+__device__ __forceinline__ void store_run_words(T* p, int n, const uint32_t (&raw)[words_of<T, N>::n]) {
     constexpr int B = N * (int)sizeof(T) >= 16 ? 16 : 8, E = B / (int)sizeof(T), W = B / 4;
-    uint32_t raw[words_of<T, N>::n];
-    f32_to_words<T, N>(v, raw);
 #pragma unroll
     for (int c = 0; c < N / E; ++c) {
         if (n >= (c + 1) * E) {
@@ -246,6 +244,14 @@ __device__ __forceinline__ void store_run_f32(T* p, int n, const float (&v)[N]) 
             }
         }
     }
+}
+
+// The same from f32 values.
+template <typename T, int N, bool NT>
+__device__ __forceinline__ void store_run_f32(T* p, int n, const float (&v)[N]) {
+    uint32_t raw[words_of<T, N>::n];
+    f32_to_words<T, N>(v, raw);
+    store_run_words<T, N, NT>(p, n, raw);
 }
 
 template <int CTRL>

@@ -105,6 +105,21 @@ def test_elementwise_launch_bounds(dev, dtype, n, off):
     same(x, want, "swiglu in place")
 
 
+# Half GELU at the bounds of its table kernel's trips on a 256-CU device (2^21, 2^22, 2^23 elements).
+@pytest.mark.parametrize("dtype", DTYPES[1:], ids=DT_ID)
+@pytest.mark.parametrize("n", [1 << 21, (1 << 21) + 1, (1 << 22) - 7, (1 << 22) + 8, 1 << 23, (1 << 23) + 9])
+def test_half_gelu_trip_bounds(dev, dtype, n):
+    print(f"case half gelu {dtype} n {n}", flush=True)
+    for off in (0, 3):
+        x = _gen((n,), 14, dev, dtype, off, 2.0)
+        for fn in (ops.gelu_tanh, ops.gelu_erf):
+            want = _pieces(fn, x)
+            assert torch.equal(fn(x).view(torch.uint8), want.view(torch.uint8))
+        y = x.clone()
+        assert ops.gelu_erf(y, out=y) is y  # in place
+        assert torch.equal(y.view(torch.uint8), want.view(torch.uint8))
+
+
 @pytest.mark.parametrize("dtype", DTYPES, ids=DT_ID)
 @pytest.mark.parametrize("rows,n,off", [(3, 1, 0), (5, 7, 1), (1, 2049, 0), (1100, 1001, 0), (1100, 1001, 1), (1048, 1000, 1),
                                         (2049, 2048, 3), (700, 4097, 0), (4000, 9001, 0)])
