@@ -348,8 +348,85 @@ __global__ __launch_bounds__(kThreads) void embed_q4_k_staged(const uint8_t* __r
     }
 }
 
+// The same for launches that the kernel above leaves short of waves or of blocks to follow one
+// another: a wave takes `per` super-blocks of a row (at most a chunk), and the rows' parts are items
+// of their own. A wave's bytes stay in its own LDS, so nothing but the wave's own order is waited for.
+// At 4096 wide, per launch, replayed back to back (one row per wave, 16 waves a block, before): 1 id
+// 3.4 -> 1.9 us, 64 5.7 -> 2.1, 333 5.8 -> 2.8, 1024 6.8 -> 4.5, 4096 14.4 -> 12.5, 16384 49.2 -> 45.4; but
+// 65536 185 -> 195. One, four and eight waves a block measured within 0.1 us up to 4096 ids and 1-5 us
+// slower at 16384; cached stores level up to 64 ids and slower beyond.
+constexpr int kPartWaves = 2;
+
+// Orders a wave's LDS stores before its later loads (LDS serves a wave in order; the compiler must not swap them).
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+__global__ __launch_bounds__(kPartWaves * kWave) void embed_q4_k_parts(const uint8_t* __restrict__ table, int64_t vocab,
+                                                                      int hidden, int64_t row_bytes,
+                                                                      const uint32_t* __restrict__ ids, uint32_t items,
+                                                                      uint32_t parts, int per, float* __restrict__ out,
+                                                                      int32_t* bad_id_flag) {
+    __shared__ __align__(16) uint8_t stage[kPartWaves][kQ4kChunkBytes];
+    const int lane = threadIdx.x & (kWave - 1);
+    const int wv = threadIdx.x / kWave;
+    const uint32_t item = __builtin_amdgcn_readfirstlane(blockIdx.x * kPartWaves + wv);
+    if (item >= items) return;
+    const uint32_t t = item / parts;
+    const int nblk = hidden / 256, c0 = (int)(item - t * parts) * per;  // the part's first super-block
+    const int nb = nblk - c0 < per ? nblk - c0 : per;
+    const uint32_t id = ids[t];
+    float* dst = out + (size_t)t * (size_t)hidden + 256 * c0 + 4 * lane;
+    if ((int64_t)id >= vocab) {
+        for (int j = 0; j < nb; ++j) store4(dst + 256 * j, 0.f, 0.f, 0.f, 0.f);
+        if (lane == 0 && bad_id_flag != nullptr) *bad_id_flag = 1;
+        return;
+    }
+    const uint8_t* src = table + (size_t)id * (size_t)row_bytes + (size_t)c0 * 144;
+    uint8_t* buf = stage[wv];
+    constexpr int kLoads = (kQ4kChunkBytes + 16 * kWave - 1) / (16 * kWave);
+    u32x4 v[kLoads];
+#pragma unroll
+    for (int k = 0; k < kLoads; ++k) {
+        const int o = (k * kWave + lane) * 16;
+        if (o < nb * 144) v[k] = *reinterpret_cast<const u32x4*>(src + o);
+    }
+#pragma unroll
+    for (int k = 0; k < kLoads; ++k) {
+        const int o = (k * kWave + lane) * 16;
+        if (o < nb * 144) *reinterpret_cast<u32x4*>(buf + o) = v[k];
+    }
+    wave_lds_sync();
+    const int qoff = 16 + 32 * (lane >> 4) + 4 * (lane & 7);  // this lane's nibble dword in a block
+    for (int j = 0; j < nb; ++j) {
+        const uint8_t* b = buf + j * 144;
+        float o[4];
+        dequant_q4k_lane(*reinterpret_cast<const u32x4*>(b), *reinterpret_cast<const uint32_t*>(b + qoff), lane, o);
+        store4(dst + 256 * j, o[0], o[1], o[2], o[3]);
+    }
+}
+
+// Waves to aim for in a launch of few ids (ten per CU).
+constexpr int64_t kPartTarget = 2560;
+// Super-blocks up to which rows are cut into parts (256 MB of output).
+constexpr int64_t kPartBlocks = int64_t(1) << 18;
+
 int launch_q4_k_staged(const void* table, int64_t vocab, int64_t hidden, int64_t row_bytes, const uint32_t* ids,
                        int64_t n_ids, float* out, int32_t* flag, hipStream_t stream) {
+    const int64_t nblk = hidden / 256;
+    if (n_ids <= kPartBlocks / nblk) {
+        // As many super-blocks per wave as leave kPartTarget waves, at most eight (16384 ids of 4096: 45.4 us
+        // with eight, 48 with sixteen).
+        int64_t per = (n_ids * nblk + kPartTarget - 1) / kPartTarget;
+        if (per > 8) per = 8;
+        const int64_t parts = (nblk + per - 1) / per;
+        const uint32_t items = (uint32_t)(n_ids * parts);  // at most kPartBlocks
+        return launch(embed_q4_k_parts, dim3((items + kPartWaves - 1) / kPartWaves), kPartWaves * kWave, stream,
+                      static_cast<const uint8_t*>(table), vocab, (int)hidden, row_bytes, ids, items, (uint32_t)parts,
+                      (int)per, out, flag);
+    }
     constexpr int64_t kChunk = int64_t(1) << 24;  // tokens per launch
     for (int64_t t0 = 0; t0 < n_ids; t0 += kChunk) {
         const int64_t nt = n_ids - t0 < kChunk ? n_ids - t0 : kChunk;

@@ -334,3 +334,24 @@ def test_embed_every_format_every_staging_width(dev, orc, fmt, hidden, offset):
     assert flag.item() == 1
     assert (out[~ok] == 0).all()
     assert_bits_equal(out[ok], orc.embed_tokens(blocks, dt, vocab, hidden, ids[ok]), f"{fmt} {hidden} +{offset}")
+
+
+# Q4_K rows cut into parts: one super-block per row and many, part lengths that the row is no multiple of (17
+# super-blocks), launches at the wave target (2560) and one past it, and past the bound of the parts (2^18 super-blocks).
+@pytest.mark.parametrize("hidden,n", [(256, 1), (256, 2560), (256, 2561), (4352, 1), (4352, 150), (4352, 333),
+                                      (4352, 2000), (4096, 16384), (4096, 16385)])
+def test_embed_q4_k_rows_in_parts(dev, orc, hidden, n):
+    vocab = 40
+    rng = np.random.default_rng(hidden + n)
+    nb = vocab * hidden // 256
+    blocks = rng.integers(0, 256, (nb, 144), dtype=np.uint8)
+    blocks[:, :4] = np.frombuffer(rng.uniform(-0.05, 0.05, 2 * nb).astype(np.float16).tobytes(), np.uint8).reshape(nb, 4)
+    ids = rng.integers(0, vocab, n).astype(np.uint32)
+    if n > 1:
+        ids[n // 2] = vocab
+    flag = torch.zeros(1, dtype=torch.int32, device=dev)
+    print(f"case embed q4_k parts hidden {hidden} ids {n}", flush=True)
+    out = to_np(ops.embed(_dev_bytes(blocks, dev), Q4_K, vocab, hidden, _ids(ids, dev), bad_id_flag=flag))
+    assert flag.item() == (n > 1)
+    rows = orc.embed_tokens(blocks, Q4_K, vocab, hidden, np.arange(vocab, dtype=np.uint32))
+    assert_bits_equal(out, np.concatenate([rows, np.zeros((1, hidden), np.float32)])[ids], f"q4_k {hidden} x {n}")
