@@ -21,7 +21,8 @@
 // Design (write-dominated: 16 KiB of f32 out per 2.3 KiB Q4_K row in):
 //  - One wave64 per token (16 tokens per 1024-thread block; 8 per 512-thread
 //    block in embed_staged, whose LDS footprint that keeps small, and 2 per
-//    block when there are too few ids to give every CU a block); each lane produces
+//    block when there are too few ids to give every CU a block; Q4_K up to
+//    256 MB of output cuts rows into parts, embed_q4_k_parts); each lane produces
 //    4 consecutive outputs per step, so every store instruction writes 1 KiB
 //    contiguous (16 bytes per lane), non-temporal (non-temporal stores and the
 //    larger block measured 4.8 → 6.5 TB/s on the Q4_K gather).
