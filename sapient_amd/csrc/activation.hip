@@ -601,8 +601,8 @@ int launch_bias(const void* y, const void* bias, void* out, int64_t total, int64
         const int tile = nvr >= kThreads ? kThreads : (int)((nvr + 63) / 64 * 64);
         const int ntiles = (int)((nvr + tile - 1) / tile);
         const int64_t groups = (rows + kBiasRowsPerBlock - 1) / kBiasRowsPerBlock;
-        // The grid is one launch: ntiles · groups < 2^32 blocks is checked here.
-        if ((int64_t)ntiles * groups < ((int64_t)1 << 31)) {
+        // The grid is one launch, of fewer than 2^32 work-items.
+        if ((int64_t)ntiles * tile <= UINT32_MAX / groups) {
             auto go = [&](auto p) {
                 constexpr int P = decltype(p)::value;
                 const dim3 grid((unsigned)(ntiles * groups));

@@ -1,0 +1,56 @@
+"""CPU: the launches of C ABI calls at sizes no test machine's memory has to hold. The library runs in a child
+process under tests/native/launch_recorder.cpp, which stands in for the HIP runtime: it refuses a launch as HIP does
+(2^32 work-items and more) and names the kernel, grid and block of every other. Nothing is run, so the pointers are
+addresses of nothing."""
+import json
+import subprocess
+import sys
+from pathlib import Path
+
+import pytest
+
+ROOT = Path(__file__).resolve().parents[1]
+RECORDER = ROOT / "tests" / "native" / "_build" / "launch_recorder.so"
+CHILD = """
+import ctypes, json, sys
+rec = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)  # before the library: its symbols come first
+rec.take_launches.restype = ctypes.c_char_p
+from sapient_amd._lib import lib
+for name, args in json.load(sys.stdin):
+    st = getattr(lib(), name)(*args)
+    print(json.dumps([st, [l.split() for l in rec.take_launches().decode().splitlines()]]))
+"""
+F32, F16 = 0, 1
+A, B, C, D, E, G, H, I = ((i + 1) << 42 for i in range(8))  # 16-byte aligned, 4 TiB apart
+
+
+@pytest.fixture(scope="module")
+def launches():
+    """launches(*calls): (status, [(kernel, grid x, grid y, block x)]) of each (function, *arguments)."""
+    import sapient_amd
+    if not sapient_amd.LIB_PATH.exists():
+        from sapient_amd import build
+        build.build()
+    if not RECORDER.exists():
+        import importlib.util
+        spec = importlib.util.spec_from_file_location("native_build", RECORDER.parents[1] / "build.py")
+        mod = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(mod)
+        mod.build()
+
+    def go(*calls):
+        res = subprocess.run([sys.executable, "-c", CHILD, str(RECORDER)], input=json.dumps([[c[0], c[1:]] for c in calls]),
+                             capture_output=True, text=True, cwd=ROOT, timeout=120)
+        assert res.returncode == 0, res.stderr
+        got = [json.loads(line) for line in res.stdout.splitlines()]
+        return [(st, [(k, int(x), int(y), int(b)) for k, x, y, b in ls]) for st, ls in got]
+    return go
+
+
+@pytest.mark.parametrize("n", [1, 3, 7, 8, 9, 63, 1001, 4096])
+def test_add_bias_at_any_row_count(launches, n):
+    """Narrow rows by the 2^27 and more, and the largest tensors: one launch within HIP's limit."""
+    calls = [("sph_add_bias", A + off, B, F32, C + off, dt, rows * n, n, None)
+             for dt in (F32, F16) for off in (0, 4 - 2 * dt) for rows in (1, (1 << 27) + 1, (1 << 36) // n)]
+    for call, (st, ls) in zip(calls, launches(*calls)):
+        assert st == 0 and len(ls) == 1, (call, st, ls)
