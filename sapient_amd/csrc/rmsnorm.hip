@@ -469,10 +469,10 @@ int launch_ragged_any(const TX* xp, TX* rp, TX* sp, const void* wp, const void* 
     const int64_t bytes = nr * dim * (int64_t)(sizeof(TX) * (adds(KIND) ? 3 : 1) + sizeof(TO));
     const bool nt = bytes >= kCachedBytes;
     int st = kNoShape;
-    if (few || (adds(KIND) && sizeof(TX) == 4)) {
-        st = nt ? launch_ragged<TX, TO, KIND, 1, true>(xp, rp, sp, wp, bp, wb_f32, op, nr, dim, eps, stream)
-                : launch_ragged<TX, TO, KIND, 1, false>(xp, rp, sp, wp, bp, wb_f32, op, nr, dim, eps, stream);
-    }
+    if constexpr (adds(KIND) && sizeof(TX) == 4)
+        if (nt) st = launch_ragged<TX, TO, KIND, 1, true>(xp, rp, sp, wp, bp, wb_f32, op, nr, dim, eps, stream);
+    if (!nt && (few || (adds(KIND) && sizeof(TX) == 4)))  // (a few values are never past kCachedBytes)
+        st = launch_ragged<TX, TO, KIND, 1, false>(xp, rp, sp, wp, bp, wb_f32, op, nr, dim, eps, stream);
     if (st != kNoShape) return st;
     return nt ? launch_ragged<TX, TO, KIND, 2, true>(xp, rp, sp, wp, bp, wb_f32, op, nr, dim, eps, stream)
               : launch_ragged<TX, TO, KIND, 2, false>(xp, rp, sp, wp, bp, wb_f32, op, nr, dim, eps, stream);

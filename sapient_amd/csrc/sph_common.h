@@ -175,6 +175,7 @@ typedef u32x4 u32x4_at4 __attribute__((aligned(4)));
 typedef u32x4 u32x4_at2 __attribute__((aligned(2)));
 typedef u32x2 u32x2_at4 __attribute__((aligned(4)));
 typedef u32x2 u32x2_at2 __attribute__((aligned(2)));
+typedef uint32_t u32_at2 __attribute__((aligned(2)));
 template <typename T, int BYTES> struct elem_vec;
 template <> struct elem_vec<float, 16> { typedef u32x4_at4 type; };
 template <> struct elem_vec<f16, 16> { typedef u32x4_at2 type; };
@@ -182,6 +183,41 @@ template <> struct elem_vec<bf16, 16> { typedef u32x4_at2 type; };
 template <> struct elem_vec<float, 8> { typedef u32x2_at4 type; };
 template <> struct elem_vec<f16, 8> { typedef u32x2_at2 type; };
 template <> struct elem_vec<bf16, 8> { typedef u32x2_at2 type; };
+
+// A short run of n < 8 halves (n < 4 where the run holds four): pieces of 4, 2 and 1 as n's bits say, so that
+// a run of any length is at most three accesses, in flight together. One access per half, each waited for
+// before the next, cost seven: add + RMSNorm f16 65536 x 7 33.4 us against 23.9, 65536 x 127 49.2 / 34.0.
+template <typename T, int E>
+__device__ __forceinline__ void load_halves(const T* p, int n, uint32_t (&raw)[E / 2]) {
+    const char* c = reinterpret_cast<const char*>(p);
+    u32x2 four = {0u, 0u};
+    uint32_t two = 0u, one = 0u;
+    if (E > 4 && (n & 4)) four = *reinterpret_cast<const u32x2_at2*>(c);
+    if (n & 2) two = *reinterpret_cast<const u32_at2*>(c + 2 * (n & 4));
+    if (n & 1) one = __builtin_bit_cast(uint16_t, p[n & 6]);
+    const uint32_t low = (n & 2) ? two : one, high = (n & 2) ? one : 0u;  // the words after the first four halves
+    raw[0] = (n & 4) ? four[0] : low;
+    raw[1] = (n & 4) ? four[1] : high;
+    if constexpr (E > 4) {
+        raw[2] = (n & 4) ? low : 0u;
+        raw[3] = (n & 4) ? high : 0u;
+    }
+}
+
+template <typename T, int E>
+__device__ __forceinline__ void store_halves(T* p, int n, const uint32_t (&raw)[E / 2]) {
+    char* c = reinterpret_cast<char*>(p);
+    uint32_t low = raw[0], high = raw[1];
+    if constexpr (E > 4) {
+        if (n & 4) {
+            *reinterpret_cast<u32x2_at2*>(c) = u32x2{low, high};
+            low = raw[2];
+            high = raw[3];
+        }
+    }
+    if (n & 2) *reinterpret_cast<u32_at2*>(c + 2 * (n & 4)) = low;
+    if (n & 1) p[n & 6] = __builtin_bit_cast(T, (uint16_t)((n & 2) ? high : low));
+}
 
 // The first min(n, N) of N consecutive elements as raw words, the rest zero bits; in accesses of
 // 16 bytes (8 where N elements are 8 bytes).
@@ -199,16 +235,12 @@ __device__ __forceinline__ void load_run(const T* p, int n, uint32_t (&raw)[word
             else q = *a;
 #pragma unroll
             for (int w = 0; w < W; ++w) raw[c * W + w] = q[w];
+        } else if constexpr (sizeof(T) == 2) {
+            static_assert(N == E, "one access");
+            load_halves<T, E>(p, n, raw);
         } else {
 #pragma unroll
-            for (int w = 0; w < W; ++w) raw[c * W + w] = 0u;
-#pragma unroll
-            for (int e = 0; e < E; ++e) {
-                if (c * E + e < n) {
-                    if constexpr (sizeof(T) == 4) raw[c * W + e] = __builtin_bit_cast(uint32_t, p[c * E + e]);
-                    else raw[c * W + e / 2] |= (uint32_t)__builtin_bit_cast(uint16_t, p[c * E + e]) << (16 * (e & 1));
-                }
-            }
+            for (int e = 0; e < E; ++e) raw[c * W + e] = c * E + e < n ? __builtin_bit_cast(uint32_t, p[c * E + e]) : 0u;
         }
     }
 }
@@ -234,14 +266,13 @@ __device__ __forceinline__ void store_run_words(T* p, int n, const uint32_t (&ra
             else q = u32x2{raw[c * W], raw[c * W + 1]};
             if constexpr (NT) __builtin_nontemporal_store(q, a);
             else *a = q;
+        } else if constexpr (sizeof(T) == 2) {
+            static_assert(N == E, "one access");
+            store_halves<T, E>(p, n, raw);
         } else {
 #pragma unroll
-            for (int e = 0; e < E; ++e) {
-                if (c * E + e < n) {
-                    if constexpr (sizeof(T) == 4) p[c * E + e] = __builtin_bit_cast(T, raw[c * W + e]);
-                    else p[c * E + e] = __builtin_bit_cast(T, (uint16_t)(raw[c * W + e / 2] >> (16 * (e & 1))));
-                }
-            }
+            for (int e = 0; e < E; ++e)
+                if (c * E + e < n) p[c * E + e] = __builtin_bit_cast(T, raw[c * W + e]);
         }
     }
 }

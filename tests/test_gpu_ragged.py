@@ -131,3 +131,25 @@ def test_ragged_bias(dev, orc, dtype, rows, n, off):
         got = ops.add_bias(y, b)
         # y + b in f32, rounded once
         assert torch.equal(got.view(torch.uint8), (y.float() + b.float()).to(dtype).view(torch.uint8))
+
+
+# Every length of a short last run (a run is 4 or 8 elements), alone in its row and after full runs; and what
+# lies past the tensor's end is left alone.
+@pytest.mark.parametrize("dtype", DTYPES, ids=DT_ID)
+@pytest.mark.parametrize("k", range(1, 8))
+def test_short_runs(dev, orc, dtype, k):
+    for dim, off in ((k, 0), (8 + k, 1), (248 + k, 0)):
+        test_ragged_norms(dev, orc, dtype, 3, dim, off)
+    print(f"case short runs {dtype} {k}", flush=True)
+    n = (1 << 21) + k
+    x, u = _gen((n,), 31, dev, dtype, 0, 2.0), _gen((n,), 32, dev, dtype, 0, 2.0)
+    guarded = lambda m: torch.full((m + 8,), 7.0, device=dev, dtype=dtype)
+    buf = guarded(n)
+    got = ops.add(x, u, out=buf[:n])
+    assert torch.equal(got, (x.float() + u.float()).to(dtype)) and (buf[n:] == 7).all()  # in f32, rounded once
+    for fn in (ops.swiglu, lambda a, b: ops.gelu_tanh(a)):
+        assert torch.equal(fn(x, u).view(torch.uint8), _pieces(fn, x, u).view(torch.uint8))
+    rows, w = 1100, 1000 + k
+    y, b, buf = _gen((rows, w), 33, dev, dtype), _gen((w,), 34, dev, torch.float32), guarded(rows * w)
+    got = ops.add_bias(y, b, out=buf[:rows * w].view(rows, w))
+    assert torch.equal(got, (y.float() + b).to(dtype)) and (buf[rows * w:] == 7).all()
