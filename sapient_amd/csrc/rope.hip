@@ -364,7 +364,8 @@ struct RopeKvArgs {
     int64_t seq, max_seq;
     int head_dim, half;
     int lanes, toks, heads;  // lanes per row; a block's tokens, and its heads per pass
-    int h_first;             // the launch's first head
+    int h_first;             // the launch's first head and token
+    int64_t s_first;
     float pos_scale;
     int32_t* bad;
     const float* ang;
@@ -441,7 +442,7 @@ __global__ __launch_bounds__(kThreads) void rope_kv_kernel(RopeKvArgs<T, TC> a) 
     const int rho = tid / a.lanes, lit = tid - rho * a.lanes;
     const int tl = TM ? rho / a.heads : rho % a.toks;  // neighbouring rows in memory: heads (TM), else tokens
     const int hl = TM ? rho - tl * a.heads : rho / a.toks;
-    const int64_t s0 = (int64_t)blockIdx.x * a.toks, s = s0 + tl;
+    const int64_t s0 = a.s_first + (int64_t)blockIdx.x * a.toks, s = s0 + tl;
     const bool active = rho < a.toks * a.heads && s < a.seq;
     const int h0 = a.h_first + (int)blockIdx.y * a.heads * U + hl, H = a.nq + a.nkv;
     const int i0 = lit * P;
@@ -662,8 +663,6 @@ int launch_rope_kv_p(RopeKvArgs<T, TC>& a, hipStream_t stream) {
     a.heads = rows / a.toks;
     if (small && a.heads > 2) a.heads = 2;
     if (a.heads > heads) a.heads = heads;
-    const int64_t blocks_x = (a.seq + a.toks - 1) / a.toks;
-    if (blocks_x > INT32_MAX) return SPH_EINVAL;
     const bool two = lanes >= 1 << 16;
     const bool bias = a.bias[0] != nullptr || a.bias[1] != nullptr || a.bias[2] != nullptr;
     const int tile = (two ? 2 : 1) * a.heads;  // heads per block
@@ -672,23 +671,28 @@ int launch_rope_kv_p(RopeKvArgs<T, TC>& a, hipStream_t stream) {
     const int64_t row = (int64_t)a.head_dim * (TM ? 2 : 1) * (int64_t)sizeof(T);
     const bool nt = two && a.seq * (a.nq * row + 2 * a.nkv * (int64_t)a.head_dim * (int64_t)(sizeof(T) + sizeof(TC))) >=
                                kCachedBytes;
+    // A launch: fewer than 2^32 work-items in x, at most 65535 blocks in y.
     constexpr int64_t kMaxY = 65535;
+    const int64_t most = UINT32_MAX / threads * (int64_t)a.toks;
     for (int64_t h0 = 0; h0 < heads; h0 += kMaxY * tile) {
         a.h_first = (int)h0;
         const int64_t tiles = (heads - h0 + tile - 1) / tile;
-        const dim3 grid((unsigned)blocks_x, (unsigned)(tiles < kMaxY ? tiles : kMaxY));
-        auto go = [&](auto u, auto b, auto n) {
-            return launch(rope_kv_kernel<T, TC, P, IL, TM, decltype(u)::value, decltype(b)::value, decltype(n)::value>,
-                          grid, threads, stream, a);
-        };
-        using std::false_type;
-        using std::true_type;
-        const std::integral_constant<int, 1> one;
-        const std::integral_constant<int, 2> pair;
-        const int st = !two ? (bias ? go(one, true_type{}, false_type{}) : go(one, false_type{}, false_type{}))
-                       : nt ? (bias ? go(pair, true_type{}, true_type{}) : go(pair, false_type{}, true_type{}))
-                            : (bias ? go(pair, true_type{}, false_type{}) : go(pair, false_type{}, false_type{}));
-        if (st != SPH_OK) return st;
+        for (a.s_first = 0; a.s_first < a.seq; a.s_first += most) {
+            const int64_t toks = a.seq - a.s_first < most ? a.seq - a.s_first : most;
+            const dim3 grid((unsigned)((toks + a.toks - 1) / a.toks), (unsigned)(tiles < kMaxY ? tiles : kMaxY));
+            auto go = [&](auto u, auto b, auto n) {
+                return launch(rope_kv_kernel<T, TC, P, IL, TM, decltype(u)::value, decltype(b)::value, decltype(n)::value>,
+                              grid, threads, stream, a);
+            };
+            using std::false_type;
+            using std::true_type;
+            const std::integral_constant<int, 1> one;
+            const std::integral_constant<int, 2> pair;
+            const int st = !two ? (bias ? go(one, true_type{}, false_type{}) : go(one, false_type{}, false_type{}))
+                           : nt ? (bias ? go(pair, true_type{}, true_type{}) : go(pair, false_type{}, true_type{}))
+                                : (bias ? go(pair, true_type{}, false_type{}) : go(pair, false_type{}, false_type{}));
+            if (st != SPH_OK) return st;
+        }
     }
     return SPH_OK;
 }

@@ -54,3 +54,14 @@ def test_add_bias_at_any_row_count(launches, n):
              for dt in (F32, F16) for off in (0, 4 - 2 * dt) for rows in (1, (1 << 27) + 1, (1 << 36) // n)]
     for call, (st, ls) in zip(calls, launches(*calls)):
         assert st == 0 and len(ls) == 1, (call, st, ls)
+
+
+@pytest.mark.parametrize("hd,il", [(8, 0), (64, 1), (128, 0), (512, 0)])
+def test_fused_rope_step_at_any_token_count(launches, hd, il):
+    """Chunks past what one launch holds are split by tokens, each launch as full as HIP allows."""
+    for seq in (1, (1 << 24) + 5, (1 << 33) // hd):
+        tail = [F32, il, D, seq, hd, 1e4, 1.0, E, G, F16, seq, None, None, None, F32, None, None]
+        calls = [("sph_rope_kv_append", A, 2, B, C, 1, *tail), ("sph_rope_kv_append_tokens", A, H, 2, B, C, 1, *tail)]
+        for st, ls in launches(*calls):
+            assert st == 0 and all(k.startswith("rope_kv_kernel<") for k, *_ in ls), (seq, st, ls)
+            assert len(ls) == 1 or all(x * b > (1 << 32) - 512 for _, x, _, b in ls[:-1]), ls

@@ -154,3 +154,25 @@ def test_kv_cache_update_past_the_head_chunk(dev, orc, q8):
     print(f"case kv_cache_update in place {n_kv} heads {'q8_0' if q8 else 'f16'}", flush=True)
     assert ops.kv_cache_update(src, cache, cur) == max_seq
     assert np.array_equal(to_np(cache).view(np.uint8), want.view(np.uint8))
+
+
+def test_rope_kv_append_past_one_launch_of_tokens(dev):
+    """2^24 + 5 tokens of 512 channels: two launches, split by tokens. The rows at both ends and around the split
+    equal those of a call on them alone."""
+    S, D = (1 << 24) + 5, 512
+    q = torch.zeros(1, S, D, device=dev, dtype=torch.float16)
+    none = torch.empty(0, S, D, device=dev, dtype=torch.float16)
+    cache = torch.empty(0, S, D, device=dev, dtype=torch.float16)
+    pos = torch.arange(S, dtype=torch.int32, device=dev)
+    at = [slice(0, 8), slice((1 << 24) - 9, S)]  # (a launch is of 2^24 - 1 blocks of a token each)
+    want = []
+    for i, a in enumerate(at):
+        q[:, a] = _randn(q[:, a].numel(), dev, torch.float16, 20 + i).view(q[:, a].shape)
+        part = q[:, a].clone()
+        n = part.shape[1]
+        ops.rope_kv_append(part, none[:, :n], none[:, :n], pos[a].contiguous(), 1e4, cache, cache)
+        want.append(part)
+    print(f"case rope_kv_append f16 1x{S}x{D}", flush=True)
+    ops.rope_kv_append(q, none, none, pos, 1e4, cache, cache)
+    for a, w in zip(at, want):
+        assert torch.equal(q[:, a], w)
