@@ -662,7 +662,17 @@ int launch_rope_kv_p(RopeKvArgs<T, TC>& a, hipStream_t stream) {
     if (a.toks > a.seq) a.toks = (int)a.seq;
     a.heads = rows / a.toks;
     if (small && a.heads > 2) a.heads = 2;
-    if (a.heads > heads) a.heads = heads;
+    if (a.heads > heads) {
+        a.heads = heads;
+        // Few heads: more tokens, so that the block's threads have rows (16384 tokens of 1 + 1 heads x 64: f16 13.7 ->
+        // 6.2 us, f32 7.0 -> 5.6).
+        if (!small) {
+            int t = rows / heads;
+            if (t > kMaxBlockAngles / a.half) t = kMaxBlockAngles / a.half;
+            if (t > a.seq) t = (int)a.seq;
+            if (t > a.toks) a.toks = t;
+        }
+    }
     const bool two = lanes >= 1 << 16;
     const bool bias = a.bias[0] != nullptr || a.bias[1] != nullptr || a.bias[2] != nullptr;
     const int tile = (two ? 2 : 1) * a.heads;  // heads per block

@@ -65,3 +65,12 @@ def test_fused_rope_step_at_any_token_count(launches, hd, il):
         for st, ls in launches(*calls):
             assert st == 0 and all(k.startswith("rope_kv_kernel<") for k, *_ in ls), (seq, st, ls)
             assert len(ls) == 1 or all(x * b > (1 << 32) - 512 for _, x, _, b in ls[:-1]), ls
+
+
+@pytest.mark.parametrize("heads", [1, 2, 3, 16])
+def test_fused_rope_step_fills_its_blocks(launches, heads):
+    """A 256-thread block takes 256 angles' tokens, also where few heads make few lanes of many tokens."""
+    seq, hd = 16384, 64
+    (st, [(_, x, y, b)]), = launches(("sph_rope_kv_append", A, heads - heads // 2, B, C, heads // 2, F16, 0, D, seq, hd, 1e4,
+                                      1.0, E, G, F16, seq, None, None, None, F16, None, None))
+    assert st == 0 and b == 256 and seq // x == 256 // (hd // 2), (x, y, b)
