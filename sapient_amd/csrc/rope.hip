@@ -364,7 +364,8 @@ struct RopeKvArgs {
     int64_t seq, max_seq;
     int head_dim, half;
     int lanes, toks, heads;  // lanes per row; a block's tokens, and its heads per pass
-    int h_first;             // the launch's first head and token
+    uint32_t by_lanes, by_toks, by_heads;  // 2^16 over each, rounded up (see quotient)
+    int h_first;                           // the launch's first head and token
     int64_t s_first;
     float pos_scale;
     int32_t* bad;
@@ -374,6 +375,12 @@ struct RopeKvArgs {
 };
 
 constexpr int kMaxBlockAngles = 256;  // a block's tokens times pairs
+
+// n / d for n < 256 and d <= 256, from 2^16 / d rounded up: exact, since the excess is below n · d / 2^16 < 1 of a
+// quotient's step. An integer division by an argument is some forty operations, and a decode step's threads would
+// start with three in a row (the engine's step 321 -> 310 us a token).
+__host__ __device__ constexpr uint32_t reciprocal(int d) { return (0x10000u + (uint32_t)d - 1) / (uint32_t)d; }
+__device__ __forceinline__ int quotient(int n, uint32_t rec) { return (int)((uint32_t)n * rec >> 16); }
 
 // A thread's share of a row, as it sits in memory: P pairs, in two runs of P elements at i0 and
 // half + i0 (NEOX) or one of 2P at 2 i0 (interleaved). In f32, f holds the runs one after the other.
@@ -407,19 +414,34 @@ struct PairRuns {
     }
 };
 
-// N consecutive bias values (of any float type) as f32; the launch checked their alignment.
+// N consecutive bias values (of any float type) as they sit in memory, halves in the first N / 2 words, so that
+// their loads join the rows' in flight. The first N / 2 words are loaded alike for either width: were they loaded
+// in a branch per type, each load would wait for the one before it. The launch checked the alignment.
 template <int N>
-__device__ __forceinline__ void load_bias(const void* p, int dt, int at, float (&b)[N]) {
-    if (dt == SPH_F32) {
-        load_f32<float, N>(static_cast<const float*>(p) + at, b);
-    } else if constexpr (N % 2 == 0) {
-        if (dt == SPH_F16) load_f32<f16, N>(static_cast<const f16*>(p) + at, b);
-        else load_f32<bf16, N>(static_cast<const bf16*>(p) + at, b);
-    } else {
-#pragma unroll
-        for (int i = 0; i < N; ++i)
-            b[i] = dt == SPH_F16 ? widen(static_cast<const f16*>(p)[at + i]) : widen(static_cast<const bf16*>(p)[at + i]);
+struct BiasRun {
+    static_assert(N % 2 == 0, "whole words of halves");
+    uint32_t w[2][N / 2];
+    __device__ __forceinline__ void load(const void* p, size_t at, bool f32) {
+        const float* q = reinterpret_cast<const float*>(static_cast<const char*>(p) + (at << (f32 ? 2 : 1)));
+        load_words<float, N / 2>(q, w[0]);
+        if (f32) load_words<float, N / 2>(q + N / 2, w[1]);
     }
+    __device__ __forceinline__ void to_f32(int dt, float (&b)[N]) const {
+        if (dt == SPH_F32) {
+#pragma unroll
+            for (int i = 0; i < N; ++i) b[i] = __uint_as_float(w[i / (N / 2)][i % (N / 2)]);
+        } else if (dt == SPH_F16) {
+            words_to_f32<f16, N>(w[0], b);
+        } else {
+            words_to_f32<bf16, N>(w[0], b);
+        }
+    }
+};
+
+// A thread's P supplied angles, (cos, sin) pairs at 8-byte alignment.
+template <int P>
+__device__ __forceinline__ void load_angles(const float* p, float (&ag)[2 * P]) {
+    load_run_f32<float, 2 * P, false>(p, 2 * P, ag);
 }
 
 // Fused decode step: heads [0, nq) are q rows, rotated and written to qo
@@ -438,64 +460,69 @@ template <typename T, typename TC, int P, bool INTERLEAVED, bool TM, int U, bool
 __global__ __launch_bounds__(kThreads) void rope_kv_kernel(RopeKvArgs<T, TC> a) {
     __shared__ uint32_t inv_pio4[24];
     __shared__ float cs_s[kMaxBlockAngles], sn_s[kMaxBlockAngles];
+    // All arguments are asked for here: left to the branches that use them, their scalar loads form a chain of cache
+    // misses, which a decode step waits for longer than for its rows (the engine's step, 24 launches of this: 334 ->
+    // 321 us a token).
+    asm volatile("" ::"s"(a.q), "s"(a.qo), "s"(a.k), "s"(a.v), "s"(a.kc), "s"(a.vc), "s"(a.pos), "s"(a.bias[0]),
+                 "s"(a.bias[1]), "s"(a.bias[2]), "s"(a.bias_dt), "s"(a.nq), "s"(a.nkv), "s"(a.seq), "s"(a.max_seq),
+                 "s"(a.head_dim), "s"(a.half), "s"(a.lanes), "s"(a.toks), "s"(a.heads), "s"(a.h_first), "s"(a.s_first),
+                 "s"(a.pos_scale), "s"(a.bad), "s"(a.ang), "s"((int)a.ang_by_pos), "s"(a.by_lanes), "s"(a.by_toks), "s"(a.by_heads));
     const int tid = threadIdx.x;
-    const int rho = tid / a.lanes, lit = tid - rho * a.lanes;
-    const int tl = TM ? rho / a.heads : rho % a.toks;  // neighbouring rows in memory: heads (TM), else tokens
-    const int hl = TM ? rho - tl * a.heads : rho / a.toks;
+    const int rho = quotient(tid, a.by_lanes), lit = tid - rho * a.lanes;
+    // Neighbouring rows in memory: heads (TM), else tokens.
+    const int major = quotient(rho, TM ? a.by_heads : a.by_toks), minor = rho - major * (TM ? a.heads : a.toks);
+    const int tl = TM ? major : minor, hl = TM ? minor : major;
     const int64_t s0 = a.s_first + (int64_t)blockIdx.x * a.toks, s = s0 + tl;
     const bool active = rho < a.toks * a.heads && s < a.seq;
     const int h0 = a.h_first + (int)blockIdx.y * a.heads * U + hl, H = a.nq + a.nkv;
     const int i0 = lit * P;
     using Runs = PairRuns<T, P, INTERLEAVED, NT>;
 
-    const bool eval = a.ang == nullptr;
+    const bool eval = a.ang == nullptr, per_token = !eval && !a.ang_by_pos;
     constexpr bool kOwn = P == 1;  // a thread's one angle: no exchange (3 tokens of 14 + 2 x 64: 2.87 -> 2.66 us)
-    uint32_t tab_word = 0;
-    if (eval && tid < 24) tab_word = kInvPio4.w[tid];
+    // Clamped, not predicated: a load in a branch is waited for at its end where its value is converted there.
+    auto pos_at = [&](int64_t t) { return a.pos[t < a.seq ? t : a.seq - 1]; };
+    const int32_t ps = pos_at(s);
     // Angle number tid of the block.
-    const int pair = eval && !kOwn ? tid / a.toks : 0, tk = tid - pair * a.toks;
+    const int pair = eval && !kOwn ? quotient(tid, a.by_toks) : 0, tk = tid - pair * a.toks;
     const bool has_angle = eval && !kOwn && pair < a.half;
+    const int32_t apos = kOwn ? ps : pos_at(s0 + tk);
+    uint32_t tab_word = 0;
     float den = 1.0f;
-    if (kOwn && eval && active) den = a.den.v[i0];
-    int32_t apos = 0;
-    if (has_angle) {
-        den = a.den.v[pair];
-        if (s0 + tk < a.seq) apos = a.pos[s0 + tk];
+    if (eval) {
+        tab_word = kInvPio4.w[tid < 24 ? tid : 0];
+        den = a.den.v[kOwn ? i0 : pair < a.half ? pair : 0];
     }
-    int32_t ps = 0;
-    if (active) ps = a.pos[s];
 
     // Row (head h, token s) of a [heads, seq, hd] (or, TM, [seq, heads, hd]) tensor.
     auto row_of = [&](const T* base, int heads, int h) {
         return base + (TM ? (size_t)s * (size_t)heads + (size_t)h : (size_t)h * (size_t)a.seq + (size_t)s) *
                           (size_t)a.head_dim;
     };
+    // Everything the rows need is requested before anything is waited for: the position, the angles where the
+    // caller supplies them per token, the rows and the biases of their channels.
+    float ag[2 * P];
+    if (per_token && active) load_angles<P>(a.ang + 2 * ((size_t)s * (size_t)a.half + (size_t)i0), ag);
     Runs x[U], w[U];  // the q or k row, and the v row
-    float xb[BIAS ? U : 1][2 * P], wb[BIAS ? U : 1][2 * P];  // their biases
-    auto bias_of = [&](int which, int h, float (&b)[2 * P]) {
-        if (a.bias[which] == nullptr) return;
+    using BiasRuns = BiasRun<Runs::L>[BIAS ? U : 1][Runs::R];
+    BiasRuns xb, wb;
+    auto load_bias = [&](const void* p, int h, BiasRun<Runs::L>(&b)[Runs::R]) {
+        if (p == nullptr) return;
 #pragma unroll
-        for (int r = 0; r < Runs::R; ++r) {
-            float t[Runs::L];
-            load_bias<Runs::L>(a.bias[which], a.bias_dt, h * a.head_dim + Runs::at(r, i0, a.half), t);
-#pragma unroll
-            for (int j = 0; j < Runs::L; ++j) b[r * Runs::L + j] = t[j];
-        }
+        for (int r = 0; r < Runs::R; ++r)
+            b[r].load(p, (size_t)h * (size_t)a.head_dim + (size_t)Runs::at(r, i0, a.half), a.bias_dt == SPH_F32);
     };
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         const int h = h0 + u * a.heads;
         if (active && h < H) {
-            const T* r = h < a.nq ? row_of(a.q, a.nq, h) : row_of(a.k, a.nkv, h - a.nq);
-            x[u].load(r, i0, a.half);
-            if (h >= a.nq) w[u].load(row_of(a.v, a.nkv, h - a.nq), i0, a.half);
+            const bool is_q = h < a.nq;
+            const int hi = is_q ? h : h - a.nq;
+            x[u].load(is_q ? row_of(a.q, a.nq, hi) : row_of(a.k, a.nkv, hi), i0, a.half);
+            if (!is_q) w[u].load(row_of(a.v, a.nkv, hi), i0, a.half);
             if constexpr (BIAS) {
-                if (h < a.nq) {
-                    bias_of(0, h, xb[u]);
-                } else {
-                    bias_of(1, h - a.nq, xb[u]);
-                    bias_of(2, h - a.nq, wb[u]);
-                }
+                load_bias(is_q ? a.bias[0] : a.bias[1], hi, xb[u]);
+                if (!is_q) load_bias(a.bias[2], hi, wb[u]);
             }
         }
     }
@@ -518,12 +545,11 @@ __global__ __launch_bounds__(kThreads) void rope_kv_kernel(RopeKvArgs<T, TC> a) 
         }
     } else {
         // Angles supplied as (cos, sin) per (token, pair), or per position in a
-        // table of max_seq rows. A position outside the table reads no row: q is
+        // table of max_seq rows. A position outside the table reads row 0 and drops it: q is
         // rotated by angle 0 (cos 1, sin 0), the caches are left alone and the flag set.
         if (!active) return;
-        const bool in_table = !a.ang_by_pos || (ps >= 0 && (int64_t)ps < a.max_seq);
-        const int64_t row = a.ang_by_pos ? (in_table ? ps : 0) : s;
-        const float* ag = a.ang + 2 * ((size_t)row * (size_t)a.half + (size_t)i0);
+        const bool in_table = per_token || (ps >= 0 && (int64_t)ps < a.max_seq);
+        if (!per_token) load_angles<P>(a.ang + 2 * ((size_t)(in_table ? ps : 0) * (size_t)a.half + (size_t)i0), ag);
 #pragma unroll
         for (int j = 0; j < P; ++j) {
             cs[j] = in_table ? ag[2 * j] : 1.0f;
@@ -535,11 +561,16 @@ __global__ __launch_bounds__(kThreads) void rope_kv_kernel(RopeKvArgs<T, TC> a) 
 
     // Row values with the bias of their channels added (y + b in f32, then
     // stored in the activation type before RoPE reads it: round through T).
-    auto values = [&](const Runs& raw, int which, const float (&b)[2 * P], float (&f)[2 * P]) {
+    auto values = [&](const Runs& raw, int which, const BiasRun<Runs::L>(&b)[Runs::R], float (&f)[2 * P]) {
         raw.to_f32(f);
         if (BIAS && a.bias[which] != nullptr) {
 #pragma unroll
-            for (int j = 0; j < 2 * P; ++j) f[j] = widen(narrow<T>(f[j] + b[j]));
+            for (int r = 0; r < Runs::R; ++r) {
+                float t[Runs::L];
+                b[r].to_f32(a.bias_dt, t);
+#pragma unroll
+                for (int j = 0; j < Runs::L; ++j) f[r * Runs::L + j] = widen(narrow<T>(f[r * Runs::L + j] + t[j]));
+            }
         }
     };
     auto rotate = [&](float (&f)[2 * P]) {
@@ -643,7 +674,8 @@ inline void fill_dens(DenTable& den, int half, int rotary_dim, float base) {
 
 // Launch shape, from the lanes that the rows need (one row per thread and pass):
 //  - small (up to 2^14: decode steps): blocks of one wave, so that the rows spread over the CUs, each with the
-//    angles of one token (two heads a block 2.96 us, four 3.14, one 3.00 at one token of 14 + 2 heads x 64);
+//    angles of one token (two heads a block 2.96 us, four 3.14, one 3.00 at one token of 14 + 2 heads x 64; with
+//    the angles supplied, 24 such layers in the engine's replayed step: 304-313 us a token, four 317-323, one 305-314);
 //  - up to 2^18: at most 64 angles a block, so that only some waves evaluate them, and from 2^16 on two rows
 //    per thread (512 tokens of 14 + 2 x 64 f32 4.1 us with 256 angles, 3.8 with 64; 333 of 32 + 8 x 128 bf16
 //    4.4 with one row, 4.0 with two; 64 tokens of 64 heads x 80 f16 4.4 with one, 4.8 with two);
@@ -673,6 +705,9 @@ int launch_rope_kv_p(RopeKvArgs<T, TC>& a, hipStream_t stream) {
             if (t > a.toks) a.toks = t;
         }
     }
+    a.by_lanes = reciprocal(a.lanes);
+    a.by_toks = reciprocal(a.toks);
+    a.by_heads = reciprocal(a.heads);
     const bool two = lanes >= 1 << 16;
     const bool bias = a.bias[0] != nullptr || a.bias[1] != nullptr || a.bias[2] != nullptr;
     const int tile = (two ? 2 : 1) * a.heads;  // heads per block

@@ -176,3 +176,22 @@ def test_rope_kv_append_past_one_launch_of_tokens(dev):
     ops.rope_kv_append(q, none, none, pos, 1e4, cache, cache)
     for a, w in zip(at, want):
         assert torch.equal(q[:, a], w)
+
+
+def test_rope_kv_append_biases_beyond_2g_channels(dev):
+    """One token of 2^22 + 3 heads x 512: the last heads' biases lie past element 2^31 (and the heads take several
+    launches). The first and last heads equal those of a call on them alone."""
+    H, D = (1 << 22) + 3, 512
+    q = _randn(H * D, dev, torch.float16, 30).view(H, 1, D)
+    b = _randn(H * D, dev, torch.float16, 31)
+    none, cache = torch.empty(0, 1, D, device=dev, dtype=torch.float16), torch.empty(0, 8, D, device=dev, dtype=torch.float16)
+    pos = torch.tensor([5], dtype=torch.int32, device=dev)
+    want = []
+    for a in (slice(0, 16), slice(H - 16, H)):
+        part = q[a].clone()
+        ops.rope_kv_append(part, none, none, pos, 1e4, cache, cache, bq=b.view(H, D)[a].reshape(-1))
+        want.append(part)
+    print(f"case rope_kv_append f16 {H}x1x{D} with bias", flush=True)
+    ops.rope_kv_append(q, none, none, pos, 1e4, cache, cache, bq=b)
+    for a, w in zip((slice(0, 16), slice(H - 16, H)), want):
+        assert torch.equal(q[a], w)
