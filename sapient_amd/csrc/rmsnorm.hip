@@ -517,8 +517,9 @@ int launch_rms(const void* x, void* residual, void* sum, const void* w, const vo
                         (w == nullptr || aligned(w, 16)) &&
                         (bias == nullptr || aligned(bias, 16)) && nvec <= (int64_t)kWave * 2 * VPT * 16 &&
                         dim <= INT32_MAX;
-    // A launch covers at most 2^22 rows, keeping grid x block below 2^32 work-items.
-    constexpr int64_t kChunk = int64_t(1) << 22;
+    // A launch covers at most 2^21 rows: one block a row is of up to 1024 threads, and HIP takes fewer than 2^32
+    // work-items.
+    constexpr int64_t kChunk = int64_t(1) << 21;
     for (int64_t r0 = 0; r0 < rows; r0 += kChunk) {
         const int64_t nr = rows - r0 < kChunk ? rows - r0 : kChunk;
         const size_t off = (size_t)r0 * (size_t)dim;

@@ -74,3 +74,19 @@ def test_fused_rope_step_fills_its_blocks(launches, heads):
     (st, [(_, x, y, b)]), = launches(("sph_rope_kv_append", A, heads - heads // 2, B, C, heads // 2, F16, 0, D, seq, hd, 1e4,
                                       1.0, E, G, F16, seq, None, None, None, F16, None, None))
     assert st == 0 and b == 256 and seq // x == 256 // (hd // 2), (x, y, b)
+
+
+@pytest.mark.parametrize("dt", [F32, F16])
+@pytest.mark.parametrize("dim", [7, 2049, 4096, 4097, 8193, 8200, 16383, 16384, 20001])
+def test_norms_at_any_row_count(launches, dt, dim):
+    """The widest blocks (16 waves a row) and the most rows a launch takes: each launch within HIP's limit, no row lost."""
+    rows = (1 << 22) + 3
+    w = [G, F32]
+    calls = [("sph_rms_norm", A, dt, *w, C, dt, rows, dim, 1e-5, None),
+             ("sph_layer_norm", A, dt, G, H, F32, C, dt, rows, dim, 1e-5, None),
+             ("sph_add_rms_norm", A, B, dt, *w, C, dt, rows, dim, 1e-5, None),
+             ("sph_add_rms_norm_to", A, B, D, dt, *w, C, dt, rows, dim, 1e-5, None)]
+    for call, (st, ls) in zip(calls, launches(*calls)):
+        assert st == 0, (call, st, ls)
+        if all(k.startswith("rms_rows_generic<") for k, *_ in ls):
+            assert sum(x for _, x, _, _ in ls) == rows

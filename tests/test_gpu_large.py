@@ -1,5 +1,5 @@
 """GPU: the op set where a 32-bit element index would wrap, and past the
-per-launch chunks the host code splits work into (2^22 rows for the row
+per-launch chunks the host code splits work into (2^21 rows for the row
 kernels, 2^24 tokens for the embedding gather).
 
 Tensors of 2^31 + a few elements (4 GiB of f16). Where the op has an exact
@@ -70,9 +70,9 @@ def test_rms_norm_half_beyond_2g_elements(dev, orc):
         assert ulp_diff16(to_np(y[sl]).reshape(-1), want.reshape(-1), torch.float16).max() <= 1
 
 
-@pytest.mark.parametrize("dim", [8, 7], ids=["vector", "generic"])
+@pytest.mark.parametrize("dim", [8, 7], ids=["vector", "ragged"])
 def test_rms_norm_rows_past_the_launch_chunk(dev, orc, dim):
-    """2^22 + 5 rows: two launches of the row kernel (vector path, and the generic path for dim 7)."""
+    """2^22 + 5 rows: three launches of the row kernel (vector path, and the ragged path for dim 7)."""
     rows = (1 << 22) + 5
     x = _randn(rows * dim, dev, torch.float32, 6).view(rows, dim)
     w = _randn(dim, dev, torch.float32, 7, 0.1) + 1
