@@ -23,7 +23,7 @@
 //  - The residual store is issued before the reduction, overlapping it.
 //  - Rows whose pointers or width do not allow aligned 16-byte access are held in
 //    registers too, in runs at element alignment (rms_rows_ragged); rows wider
-//    than 16 waves hold take a block-per-row two-pass kernel.
+//    than 16 waves hold, and a few narrow ones, take a block-per-row two-pass kernel.
 //
 // Parity: x·x, the division by dim, sqrt and 1/· are IEEE-rounded f32 exactly
 // as in the reference; the products y = (r·inv)·w round in the same order (the
@@ -494,8 +494,9 @@ int launch_ragged_any(const TX* xp, TX* rp, TX* sp, const void* wp, const void* 
 //    row: 92.0, 55.6).
 // A row too wide for the looping shape takes the one-block-per-row kernel
 // (twice the values per lane past 16 waves); rows without aligned 16-byte access
-// the ragged kernel, and rows wider than that the generic kernel.
+// the ragged kernel, and rows wider than that, or a few narrow ones, the generic kernel.
 constexpr int64_t kFewValues = int64_t(1) << 21;
+constexpr int64_t kFewElems = int64_t(1) << 18;
 
 template <typename TX, typename TW, typename TO, int KIND>
 int launch_rms(const void* x, void* residual, void* sum, const void* w, const void* bias, void* out, int64_t rows,
@@ -550,9 +551,15 @@ int launch_rms(const void* x, void* residual, void* sum, const void* w, const vo
                 st = launch_shape<TX, TW, TO, KIND, 2 * VPT, false>(xp, rp, sp, wp, bp, op, nr, (int)dim, eps, 16, stream);
             if (st == kNoShape) return SPH_EINVAL;  // unreachable: vec_ok bounds the width
         } else {
-            st = launch_ragged_any<TX, TO, KIND>(xp, rp, sp, w, bias, std::is_same<TW, float>::value, op, nr, dim, eps,
-                                                 nr * dim <= kFewValues, stream);
-            if (st == kNoShape)  // wider than 16 waves at two runs per lane
+            // A few narrow rows stay with the kernel of element accesses, a chain of single loads: one row's waves
+            // have no more than that to do, and short runs and conversions are a longer one. Halves 300 x 127 add +
+            // RMSNorm 2.9 us against 3.6 ragged, 300 x 17 2.85 / 3.8, LayerNorm 2.6 / 3.5, 1024 x 255 RMSNorm 2.75 /
+            // 2.85, but 4096 x 127 4.9 / 4.8, 300 x 513 3.9 / 3.5; f32 300 x 17 2.35 / 2.65, 300 x 65 2.44 / 2.5.
+            const bool narrow = nr <= 3072 && dim < (HALF ? 512 : 64) && nr * dim <= kFewElems;
+            if (!narrow)
+                st = launch_ragged_any<TX, TO, KIND>(xp, rp, sp, w, bias, std::is_same<TW, float>::value, op, nr, dim,
+                                                     eps, nr * dim <= kFewValues, stream);
+            if (st == kNoShape)  // or wider than 16 waves at two runs per lane
                 st = launch(rms_rows_generic<TX, TW, TO, KIND>, dim3((unsigned)nr), 256, stream, xp, rp, sp, wp, bp, op,
                             nr, dim, eps);
         }

@@ -90,3 +90,15 @@ def test_norms_at_any_row_count(launches, dt, dim):
         assert st == 0, (call, st, ls)
         if all(k.startswith("rms_rows_generic<") for k, *_ in ls):
             assert sum(x for _, x, _, _ in ls) == rows
+
+
+# The kernel of element accesses is the quicker one for a few narrow rows, the ragged one from there on.
+@pytest.mark.parametrize("dt,rows,dim,kernel", [(F16, 1, 7, "generic"), (F16, 300, 127, "generic"), (F16, 514, 511, "ragged"),
+                                                (F16, 3073, 7, "ragged"), (F16, 2100, 127, "ragged"), (F16, 1, 513, "ragged"), (F32, 300, 17, "generic"),
+                                                (F32, 1, 65, "ragged"), (F32, 3073, 7, "ragged")])
+def test_few_narrow_norm_rows(launches, dt, rows, dim, kernel):
+    for call in (("sph_rms_norm", A, dt, G, F32, C, dt, rows, dim, 1e-5, None),
+                 ("sph_add_rms_norm", A, B, dt, G, dt, C, F32, rows, dim, 1e-5, None),
+                 ("sph_layer_norm", A, dt, G, H, F32, C, dt, rows, dim, 1e-5, None)):
+        (st, [(k, *_)]), = launches(call)
+        assert st == 0 and k.startswith(f"rms_rows_{kernel}<"), k

@@ -41,11 +41,13 @@ def _close(got, want32, orc, what):
 
 
 # One element; a run of 8 / 4 and one either side; one and two waves' spans; 16 waves at one and at two
-# runs per lane (f32 4096 / 8192, halves 8192 / 16384) and one past them; 65536 x 515: past the cached bound.
+# runs per lane (f32 4096 / 8192, halves 8192 / 16384) and one past them; 65536 x 515: past the cached bound; narrow
+# rows both few (the kernel of element accesses) and more than 3072.
 @pytest.mark.parametrize("dtype", DTYPES, ids=DT_ID)
 @pytest.mark.parametrize("rows,dim,off", [(3, 1, 0), (5, 7, 0), (5, 9, 1), (4, 255, 0), (4, 257, 0), (3, 513, 3),
                                           (700, 1025, 0), (2100, 1023, 0), (5, 4095, 0), (5, 4097, 1), (3, 8191, 0),
-                                          (3, 8193, 0), (2, 16383, 0), (2, 16385, 0), (65536, 515, 0), (9, 512, 1)])
+                                          (3, 8193, 0), (2, 16383, 0), (2, 16385, 0), (65536, 515, 0), (9, 512, 1),
+                                          (3073, 1, 0), (3073, 7, 1), (3073, 9, 0), (3073, 255, 1), (3073, 257, 0)])
 def test_ragged_norms(dev, orc, dtype, rows, dim, off):
     print(f"case ragged norms {dtype} {rows}x{dim} offset {off}", flush=True)
     x = _gen((rows, dim), 1, dev, dtype, off, mean=0.25)
@@ -139,7 +141,7 @@ def test_ragged_bias(dev, orc, dtype, rows, n, off):
 @pytest.mark.parametrize("k", range(1, 8))
 def test_short_runs(dev, orc, dtype, k):
     for dim, off in ((k, 0), (8 + k, 1), (248 + k, 0)):
-        test_ragged_norms(dev, orc, dtype, 3, dim, off)
+        test_ragged_norms(dev, orc, dtype, 3073, dim, off)  # (fewer narrow rows take the element kernel)
     print(f"case short runs {dtype} {k}", flush=True)
     n = (1 << 21) + k
     x, u = _gen((n,), 31, dev, dtype, 0, 2.0), _gen((n,), 32, dev, dtype, 0, 2.0)
