@@ -577,7 +577,7 @@ __global__ __launch_bounds__(kThreads) void bias_rows(const T* y, const TB* bias
     }
 }
 
-// Rows too wide or too many for that grid, and small ragged launches: element-wise, one modulo per element.
+// Rows too wide or too many for that grid, and small or narrow ragged launches: element-wise, one modulo per element.
 template <typename T, typename TB>
 __global__ __launch_bounds__(kThreads) void bias_scalar(const T* y, const TB* bias, T* out, int64_t total, int64_t n) {
     const int64_t stride = (int64_t)gridDim.x * kThreads;
@@ -593,11 +593,14 @@ int launch_bias(const void* y, const void* bias, void* out, int64_t total, int64
     T* op = static_cast<T*>(out);
     const int64_t rows = total / n;
     const int64_t nvr = (n + E - 1) / E;
-    // Small launches whose rows no aligned vector fits: bf16 500 x 1001 2.4 µs element by element
-    // against 3.1 in runs, 1000 x 1001 3.0 / 3.3, 2000 x 1001 4.1 / 3.7.
-    const bool few = total <= (int64_t)1 << 20 &&
-                     !(n % E == 0 && aligned(y, 16) && aligned(out, 16) && aligned(bias, 16));
-    if (!few && nvr <= (int64_t)1 << 24) {
+    // Launches whose rows no aligned vector fits go element by element while they are small (bf16 500 x 1001 2.4 µs
+    // against 3.1 in runs, 1000 x 1001 3.0 / 3.3, 2000 x 1001 4.1 / 3.7) or their rows narrow: a block holds two rows,
+    // so few of its threads have a run. f32 16M / n x n: n = 1 31 µs against 1769 in runs, 63 31 / 41, 129 31 / 28,
+    // 257 31 / 24 (at 2M, 129 4.8 / 5.7, 255 4.8 / 5.9, 257 4.8 / 4.5); f16 1 29 / 2035, 127 28 / 30 (at 64M
+    // 76 / 135), 257 27 / 17 (at 64M 76 / 87), 300 27 / 14 (75 / 64).
+    const bool by_element = !(n % E == 0 && aligned(y, 16) && aligned(out, 16) && aligned(bias, 16)) &&
+                            (total <= (int64_t)1 << 20 || n <= (sizeof(T) == 2 ? 288 : 256));
+    if (!by_element && nvr <= (int64_t)1 << 24) {
         const int tile = nvr >= kThreads ? kThreads : (int)((nvr + 63) / 64 * 64);
         const int ntiles = (int)((nvr + tile - 1) / tile);
         const int64_t groups = (rows + kBiasRowsPerBlock - 1) / kBiasRowsPerBlock;

@@ -102,3 +102,14 @@ def test_few_narrow_norm_rows(launches, dt, rows, dim, kernel):
                  ("sph_layer_norm", A, dt, G, H, F32, C, dt, rows, dim, 1e-5, None)):
         (st, [(k, *_)]), = launches(call)
         assert st == 0 and k.startswith(f"rms_rows_{kernel}<"), k
+
+
+# Rows no aligned vector fits: element by element in small launches and where they are narrow, else in runs.
+@pytest.mark.parametrize("dt,off,total,n,kernel", [(F32, 0, 1 << 24, 1, "scalar"), (F32, 0, 1 << 24, 255, "scalar"),
+                                                   (F32, 4, 1 << 24, 256, "scalar"), (F32, 0, 1 << 24, 257, "rows"),
+                                                   (F16, 0, 1 << 24, 7, "scalar"), (F16, 2, 1 << 24, 288, "scalar"),
+                                                   (F16, 0, 1 << 24, 289, "rows"), (F16, 0, 1 << 20, 1001, "scalar"),
+                                                   (F16, 0, 1 << 20, 1000, "rows")])
+def test_ragged_bias_kernel(launches, dt, off, total, n, kernel):
+    (st, [(k, *_)]), = launches(("sph_add_bias", A + off, B, F32, C + off, dt, total // n * n, n, None))
+    assert st == 0 and k.startswith(f"bias_{kernel}<"), k

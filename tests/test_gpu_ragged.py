@@ -124,7 +124,8 @@ def test_half_gelu_trip_bounds(dev, dtype, n):
 
 @pytest.mark.parametrize("dtype", DTYPES, ids=DT_ID)
 @pytest.mark.parametrize("rows,n,off", [(3, 1, 0), (5, 7, 1), (1, 2049, 0), (1100, 1001, 0), (1100, 1001, 1), (1048, 1000, 1),
-                                        (2049, 2048, 3), (700, 4097, 0), (4000, 9001, 0)])
+                                        (2049, 2048, 3), (700, 4097, 0), (4000, 9001, 0), (1100000, 1, 0), (400001, 3, 1),
+                                        (200000, 7, 0), (150000, 9, 1), (5000, 256, 1), (5000, 257, 0), (5000, 289, 0)])
 def test_ragged_bias(dev, orc, dtype, rows, n, off):
     print(f"case ragged bias {dtype} {rows}x{n} offset {off}", flush=True)
     y = _gen((rows, n), 21, dev, dtype, off)
