@@ -113,3 +113,13 @@ def test_few_narrow_norm_rows(launches, dt, rows, dim, kernel):
 def test_ragged_bias_kernel(launches, dt, off, total, n, kernel):
     (st, [(k, *_)]), = launches(("sph_add_bias", A + off, B, F32, C + off, dt, total // n * n, n, None))
     assert st == 0 and k.startswith(f"bias_{kernel}<"), k
+
+
+# Half GELU: single elements in small launches, and longer at addresses without 16-byte alignment.
+@pytest.mark.parametrize("off,n,kernel", [(0, 1 << 18, "_scalar"), (0, (1 << 18) + 8, ""), (2, (1 << 18) + 1, "_scalar"),
+                                          (8, 9 << 18, "_scalar"), (2, (9 << 18) + 1, "")])
+@pytest.mark.parametrize("fn", ["sph_gelu_tanh", "sph_gelu_erf"])
+def test_half_gelu_kernel(launches, fn, off, n, kernel):
+    for a, c in ((A + off, C), (A, C + off)):
+        (st, ls), = launches((fn, a, c, F16, n, None))
+        assert st == 0 and ls[-1][0].startswith(f"gelu_lut_apply{kernel}<"), ls[-1]  # (the first call builds the tables)

@@ -107,9 +107,10 @@ def test_elementwise_launch_bounds(dev, dtype, n, off):
     same(x, want, "swiglu in place")
 
 
-# Half GELU at the bounds of its table kernel's trips on a 256-CU device (2^21, 2^22, 2^23 elements).
+# Half GELU at the bounds of its table kernel's trips on a 256-CU device (2^21, 2^22, 2^23 elements), and of the
+# element kernel's sizes (2^18; 9 x 2^18 at unaligned addresses).
 @pytest.mark.parametrize("dtype", DTYPES[1:], ids=DT_ID)
-@pytest.mark.parametrize("n", [1 << 21, (1 << 21) + 1, (1 << 22) - 7, (1 << 22) + 8, 1 << 23, (1 << 23) + 9])
+@pytest.mark.parametrize("n", [(1 << 18) + 1, (9 << 18) + 1, 1 << 21, (1 << 21) + 1, (1 << 22) - 7, (1 << 22) + 8, 1 << 23, (1 << 23) + 9])
 def test_half_gelu_trip_bounds(dev, dtype, n):
     print(f"case half gelu {dtype} n {n}", flush=True)
     for off in (0, 3):
