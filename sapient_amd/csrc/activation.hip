@@ -298,10 +298,7 @@ int launch_ew(const void* a, const void* b, void* out, int64_t n, hipStream_t st
     if constexpr (kHalfLong)
         if (n <= kFewElems << 3) return go(std::integral_constant<int, 4>{}, one, cached);
     if ((n + E - 1) / E <= kFewVecs) return policy == P_CACHED ? go(run, one, cached) : go(run, one, nt_stores);
-    // Adds and products do too little per element to gain from cached loads of operands past the L2s: f32 x · scalar of
-    // 67 MB 8.0 µs non-temporal against 10.3, f16 a + b of 63 MB 8.0 / 10.2, f32 of 75 MB 10.9 / 12.1.
-    if constexpr (OP == OP_ADD || OP == OP_MUL) return go(run, two, nt);
-    else return policy == P_NT ? go(run, two, nt) : go(run, two, nt_stores);
+    return policy == P_NT ? go(run, two, nt) : go(run, two, nt_stores);
 }
 
 template <int OP>

@@ -123,14 +123,3 @@ def test_half_gelu_kernel(launches, fn, off, n, kernel):
     for a, c in ((A + off, C), (A, C + off)):
         (st, ls), = launches((fn, a, c, F16, n, None))
         assert st == 0 and ls[-1][0].startswith(f"gelu_lut_apply{kernel}<"), ls[-1]  # (the first call builds the tables)
-
-
-# Launches past 2^20 vectors of 16 bytes: adds and products pass the caches by (policy 2), SwiGLU and SiLU below
-# 128 MB of traffic with their stores only (policy 1).
-def test_element_wise_cache_policy(launches):
-    n = (1 << 22) + 4
-    calls = [("sph_add", A, n, B, n, C, F32, None), ("sph_mul", A, 2 * n, B, 1, C, F16, None),
-             ("sph_mul", A, 1, B, n, C, F32, None), ("sph_silu", A, C, F32, n, None), ("sph_swiglu", A, B, C, F32, n, None)]
-    for call, want in zip(calls, (2, 2, 2, 1, 1)):
-        (st, [(k, *_)]), = launches(call)
-        assert st == 0 and int(k.split(",")[5]) == want, k
