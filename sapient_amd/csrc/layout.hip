@@ -209,7 +209,7 @@ __global__ __launch_bounds__(kThreads) void kv_append_q8_0(const TS* __restrict_
 // on its own — no ordering between blocks, no scratch memory — and the kernel
 // boundary orders the two passes; the second writes the new rows too where the cache's
 // rows split into 16-byte units (kv_reverse_append: f16 2 x 4096 x 64 7.7 -> 5.4 us, a launch
-// less). Shifts of a few rows move in windows instead (Windows). Each pass reads and writes every row once
+// less). Shifts of a few rows of a larger cache move in windows instead (Windows). Each pass reads and writes every row once
 // (twice the bytes of a direct move) in whole rows, coalesced, over the whole
 // GPU; a direct in-place move must keep each column of a head in one block,
 // since a row is read by the row `shift` below it (16 bytes per row access,
@@ -249,8 +249,8 @@ int launch_reverse(void* cache, uint64_t n_heads, uint64_t row_bytes, uint64_t m
     return SPH_OK;
 }
 
-// The shift of a few rows (decode steps), each row moved once, in two launches. The rows [0, cur_len) of a
-// head are cut into windows.
+// The shift of a few rows (decode steps) in two launches: each row moves once, and `shift` rows of every window
+// a second time. The rows [0, cur_len) of a head are cut into windows.
 //  1. Every window's first `shift` rows (its slot) take the next window's: those are the rows that follow
 //     the window, and the rows a slot held are the ones that the window before it takes. (The first slot's
 //     rows are the dropped ones.)
@@ -258,10 +258,10 @@ int launch_reverse(void* cache, uint64_t n_heads, uint64_t row_bytes, uint64_t m
 //     end is the new rows' place.
 // A block holds all it moves in registers between its loads and its stores, so the in-place moves need no
 // order between blocks; only the two launches are ordered. HBM-bound: the second launch moves 33.5 MB in
-// 5.5-7.5 us, the first waits on memory once (1.6-2.7 us). A one-token update against the two reversal
-// passes and the append, in turn on one MI355X: f16 8 x 8192 x 128 12.6 -> 10.0 us, 32 x 4096 x 80 16.1 ->
-// 10.7, 8 x 32768 x 128 42.3 -> 25.3, 2 x 4096 x 64 8.7 -> 6.1; f32 8 x 8192 x 128 33.2 -> 16.6; Q8_0
-// 8 x 8192 x 128 11.2 -> 10.6. Non-temporal accesses cost 1-3 us.
+// 5.5-7.5 us, the first waits on memory once (1.6-2.7 us). A one-token update against the reversal with its
+// append, in turn on one MI355X: f16 32 x 4096 x 96 13.2 -> 10.7 us, 8 x 16384 x 128 20.8 -> 14.5; f32 31.3 -> 18.9,
+// 38.8 -> 25.5; Q8_0 20.9 -> 15.6, 13.8 -> 12.8. Non-temporal accesses cost 1-3 us. Caches below kWindowBytes are
+// bound by latency, the slots' launch above all, and reverse.
 struct Windows {
     uint32_t count, shift;
     uint32_t step, rem;  // window c starts at row c * step + min(c, rem)
@@ -351,13 +351,22 @@ __global__ __launch_bounds__(kThreads) void kv_rotate_append(TD* cache, const TS
     }
 }
 
+// Valid rows (bytes, all heads) from which a cache that is cut into windows slides faster so than by reversal, by
+// shift: f16 2 x 4096 x 64 (1 MB) 1 row 5.0 us against 4.5, 4 5.2 / 4.4, 16 7.0 / 4.6; 8 x 2048 x 128 (4.2 MB) 5.5 /
+// 5.3, 6.4 / 5.6, 7.7 / 6.4; 8 x 4096 x 128 (8.4 MB) 6.3 / 6.9, 8.1 / 7.0, 9.1 / 9.0; 40 x 4000 x 32 (10 MB) 6.5 /
+// 7.6, 6.7 / 7.8, 7.0 / 8.1; Q8_0 8 x 4096 x 128 (4.5 MB) 8.1 / 7.8, 9.7 / 8.4, 10.1 / 9.5; 40 x 4000 x 32 (5.4 MB)
+// 9.7 / 11.9, 11.3 / 12.3, 12.6 / 13.9. (8 MB at 4-8 rows, the reversal's by 1 us, is still the faster for what the
+// two passes and the append took.) A head that one block holds has no slots: one launch, 2.3 us against 3.6.
+constexpr uint64_t kWindowBytes = (uint64_t)5 << 20;
+
 // The window cut for a shift; count = 0 where it does not apply: a window has to hold twice the shift, so
 // that the slots' extra move stays well below the second move of every row that the reversal makes.
-inline Windows cut_windows(uint64_t cur_len, uint64_t shift, uint64_t upr) {
+inline Windows cut_windows(uint64_t n_heads, uint64_t cur_len, uint64_t shift, uint64_t upr, uint64_t unit) {
     const uint64_t most = upr == 0 ? 0 : (uint64_t)kRotateUnits * kThreads / upr;  // rows a block holds
     if (cur_len <= shift || cur_len > INT32_MAX || 2 * shift + 2 > most) return Windows{0, 0, 0, 0};
     const uint64_t n = (cur_len + most - 1) / most;
     if (n > kSlotThreads * kSlotUnits) return Windows{0, 0, 0, 0};
+    if (n > 1 && cur_len * upr * unit < (kWindowBytes + n_heads - 1) / n_heads) return Windows{0, 0, 0, 0};
     // n > 1: every window has at least cur_len / n > most / 2 > shift rows.
     return Windows{(uint32_t)n, (uint32_t)shift, (uint32_t)(cur_len / n), (uint32_t)(cur_len % n)};
 }
@@ -430,7 +439,7 @@ int shift_append(const void* src, void* cache, uint64_t n_heads, uint64_t hd, ui
     constexpr uint64_t E = vec16<TD>::n;
     const uint64_t upr = hd / E, keep = cur_len - shift;
     const TS* s = static_cast<const TS*>(src);
-    const Windows w = cut_windows(cur_len, shift, upr);
+    const Windows w = cut_windows(n_heads, cur_len, shift, upr, 16);
     if (w.count > 0) return shift_by_windows<u32x4, TS, TD>(cache, s, n_heads, upr, seq, max_seq, keep, w, stream);
     int st = launch_reverse<u32x4>(cache, n_heads, hd * sizeof(TD), max_seq, shift, cur_len, stream);
     if (st != SPH_OK) return st;
@@ -454,7 +463,7 @@ int shift_window(void* cache, uint64_t n_heads, uint64_t row_bytes, uint64_t max
                  uint64_t cur_len, hipStream_t stream) {
     const uint64_t upr = row_bytes / sizeof(UT);
     if (upr > UINT32_MAX || cur_len / 2 * upr > UINT32_MAX - kThreads) return SPH_EINVAL;
-    const Windows w = cut_windows(cur_len, shift, upr);
+    const Windows w = cut_windows(n_heads, cur_len, shift, upr, sizeof(UT));
     if (w.count > 0)
         return shift_by_windows<UT, void, void>(cache, nullptr, n_heads, upr, 0, max_seq, cur_len - shift, w, stream);
     const int st = launch_reverse<UT>(cache, n_heads, row_bytes, max_seq, shift, cur_len, stream);

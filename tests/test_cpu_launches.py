@@ -16,8 +16,9 @@ import ctypes, json, sys
 rec = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)  # before the library: its symbols come first
 rec.take_launches.restype = ctypes.c_char_p
 from sapient_amd._lib import lib
+n = ctypes.c_int64()
 for name, args in json.load(sys.stdin):
-    st = getattr(lib(), name)(*args)
+    st = getattr(lib(), name)(*[ctypes.addressof(n) if a == "host int64" else a for a in args])
     print(json.dumps([st, [l.split() for l in rec.take_launches().decode().splitlines()]]))
 """
 F32, F16 = 0, 1
@@ -123,3 +124,18 @@ def test_half_gelu_kernel(launches, fn, off, n, kernel):
     for a, c in ((A + off, C), (A, C + off)):
         (st, ls), = launches((fn, a, c, F16, n, None))
         assert st == 0 and ls[-1][0].startswith(f"gelu_lut_apply{kernel}<"), ls[-1]  # (the first call builds the tables)
+
+
+# An in-place slide: windows where one block holds a head, and from 5 MB of valid rows on (up to 4096 windows a head);
+# by reversal else. Float caches append in the last launch, others in a launch of their own.
+@pytest.mark.parametrize("heads,hd,dt,cur,shift,kernels", [
+    (2, 128, F16, 64, 31, ["kv_rotate_append"]), (2, 128, F16, 65, 31, ["kv_reverse_rows", "kv_reverse_append"]),
+    (2, 64, F16, 4096, 16, ["kv_reverse_rows", "kv_reverse_append"]), (8, 128, F16, 2560, 1, ["kv_shift_slots", "kv_rotate_append"]),
+    (8, 128, F16, 2559, 1, ["kv_reverse_rows", "kv_reverse_append"]), (8, 128, F16, 8192, 32, ["kv_reverse_rows", "kv_reverse_append"]),
+    (8, 128, 8, 8192, 1, ["kv_shift_slots", "kv_rotate_windows", "kv_append_q8_0"]),
+    (2, 64, 8, 4096, 4, ["kv_reverse_rows", "kv_reverse_rows", "kv_append_q8_0"]),
+    (1, 8, F16, 4096 << 10, 3, ["kv_shift_slots", "kv_rotate_append"]),
+    (1, 8, F16, (4096 << 10) + 1, 3, ["kv_reverse_rows", "kv_reverse_append"])])
+def test_kv_slide_form(launches, heads, hd, dt, cur, shift, kernels):
+    (st, ls), = launches(("sph_kv_cache_update", A, F16, B, dt, heads, shift, hd, cur, cur, "host int64", None))
+    assert st == 0 and [k.split("<")[0] for k, *_ in ls] == kernels, ls

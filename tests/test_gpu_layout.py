@@ -399,8 +399,9 @@ def test_kv_cache_update_into_rejects_bad_arguments(dev):
     assert n.value == -7 and torch.equal(cache, before) and torch.equal(out, out_before)
 
 
-# In-place slides across the launch forms. In windows: one window and two, the largest shift a window takes and
-# one more (f16 rows of 128: 31; f32: 15), more new rows than the shift, rows of each unit width, many heads.
+# In-place slides across the launch forms. In windows (one window; several from 5 MB of rows on): one window and two,
+# the largest shift a window takes and one more (f16 rows of 128: 31; f32: 15), more new rows than the shift, rows of
+# each unit width, many heads, the most windows a head takes and one more.
 # By reversal with the append: odd and even cur_len, a shift past the middle. Q8_0: the append on its own.
 @pytest.mark.parametrize("cdtype,n_kv,hd,max_seq,cur_len,seq", [
     (torch.float16, 2, 128, 64, 64, 1), (torch.float16, 2, 128, 65, 65, 1), (torch.bfloat16, 3, 64, 34, 33, 2),
@@ -409,7 +410,12 @@ def test_kv_cache_update_into_rejects_bad_arguments(dev):
     (torch.float32, 8, 128, 8191, 8190, 9), (torch.float32, 2, 128, 2000, 2000, 15), (torch.float16, 3000, 64, 60, 60, 1),
     (torch.float16, 2, 128, 300, 300, 32), (torch.bfloat16, 2, 128, 301, 300, 41), (torch.float32, 2, 128, 64, 61, 50),
     (torch.float32, 2, 128, 501, 501, 16), (torch.float16, 2, 128, 50, 50, 50),
-    (torch.uint8, 32, 128, 5000, 5000, 1), (torch.uint8, 3, 96, 701, 700, 3), (torch.uint8, 2, 64, 300, 300, 100)])
+    (torch.uint8, 32, 128, 5000, 5000, 1), (torch.uint8, 3, 96, 701, 700, 3), (torch.uint8, 2, 64, 300, 300, 100),
+    (torch.float16, 400, 128, 65, 65, 1), (torch.float16, 400, 128, 65, 65, 31), (torch.bfloat16, 700, 64, 130, 129, 40),
+    (torch.float32, 500, 8, 513, 513, 255), (torch.float16, 100, 40, 1000, 995, 20), (torch.float32, 10, 128, 2000, 2000, 15),
+    (torch.float16, 100, 36, 1000, 1000, 30), (torch.float16, 100, 38, 1000, 990, 25), (torch.float16, 100, 37, 1000, 1000, 12),
+    (torch.float16, 1, 8, 4096 << 10, 4096 << 10, 3), (torch.float16, 1, 8, (4096 << 10) + 1, (4096 << 10) + 1, 3),
+    (torch.uint8, 100, 96, 701, 700, 3)])
 def test_kv_cache_update_in_place_forms(dev, cdtype, n_kv, hd, max_seq, cur_len, seq):
     print(f"case kv_cache_update forms {cdtype} {n_kv}x{hd} max {max_seq} cur {cur_len} seq {seq}", flush=True)
     g = torch.Generator(device=dev).manual_seed(n_kv + hd)
