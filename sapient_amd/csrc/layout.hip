@@ -669,11 +669,12 @@ extern "C" int sph_kv_cache_update(const void* src, int src_dtype, void* cache, 
         if (cache == nullptr) return SPH_EINVAL;
         const uint64_t row_bytes = q8 ? (uint64_t)head_dim / 32 * 34 : (uint64_t)head_dim * sph::dtype_size(cache_dtype);
         int st;
-        // Float caches whose rows split into 16-byte units: the append rides in the shift's last launch.
+        // Float caches whose rows split into 16-byte units: the append rides in the shift's last launch (of fewer than 2^32
+        // work-items, the windows' and the rounding of both counts to blocks included).
         if (!q8 && row_bytes % 16 == 0 && sph::aligned(cache, 16)) {
             const uint64_t e = 16 / sph::dtype_size(cache_dtype), src_access = e * sph::dtype_size(src_dtype);
             if (sph::aligned(src, src_access < 16 ? src_access : 16) &&
-                ((uint64_t)cur_len / 2 + 1 + (uint64_t)seq) * ((uint64_t)head_dim / e) <= UINT32_MAX - sph::kThreads) {
+                ((uint64_t)cur_len / 2 + 1 + (uint64_t)seq) * ((uint64_t)head_dim / e) <= UINT32_MAX - 4 * sph::kThreads) {
                 st = sph::with_float_type(src_dtype, [&](auto ts) -> int {
                     using TS = decltype(ts);
                     return sph::with_float_type(cache_dtype, [&](auto td) -> int {

@@ -139,3 +139,10 @@ def test_half_gelu_kernel(launches, fn, off, n, kernel):
 def test_kv_slide_form(launches, heads, hd, dt, cur, shift, kernels):
     (st, ls), = launches(("sph_kv_cache_update", A, F16, B, dt, heads, shift, hd, cur, cur, "host int64", None))
     assert st == 0 and [k.split("<")[0] for k, *_ in ls] == kernels, ls
+
+
+def test_kv_slide_at_the_most_rows_a_launch_takes(launches):
+    """Rows past cur_len ride in the launch of the windows: within HIP's limit, else an append of its own."""
+    for seq in range((1 << 32) - 300, (1 << 32) - 256, 3):
+        (st, ls), = launches(("sph_kv_cache_update", A, F16, B, F16, 1, seq, 8, seq + 1, 2, "host int64", None))
+        assert st == 0 and ls, (seq, st)
