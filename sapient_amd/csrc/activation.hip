@@ -64,8 +64,9 @@ constexpr int64_t kFewVecs = int64_t(1) << 20;
 // the ops whose per-element work is long: a thread's chain is then one element's, and all CUs have
 // work. Half-precision SiLU and SwiGLU up to 2^19 elements, then runs of four (8 bytes) up to 2^21,
 // then of eight: bf16 SwiGLU of 0.3 M elements 2.45 / 2.76 / 3.38 µs with one / four / eight, 1 M
-// 3.63 / 3.41 / 3.72, 3 M 6.88 / 6.01 / 5.73. GELU in f32 up to 2^21 (0.3 M 2.41 µs against 3.07
-// with four, 2 M 5.64 / 5.73, 3 M 7.90 / 6.90). f32 SiLU and SwiGLU from 2048 elements up to 2^18
+// 3.63 / 3.41 / 3.72, 3 M 6.88 / 6.01 / 5.73. GELU in f32 up to 2^18 (alone 0.3 M 2.41 µs against 3.07
+// with four and 1 M level, but between the bias that wrote its input and an add, the three 0.4 M
+// 7.9 / 7.1 µs, 1 M 12.0 / 9.0, 2 M 19.7 / 13.4). f32 SiLU and SwiGLU from 2048 elements up to 2^18
 // (0.3 M 2.35 / 2.5, 1 M 3.70 / 3.39; below 2048 level or 0.3 % slower); adds and products never
 // gain. Half-precision GELU reads its table from cache up to kFewElems instead of staging it per
 // block (1 x 10240 f16 2.90 -> 1.79 µs). Results are the same bits either way.
@@ -277,8 +278,11 @@ int launch_ew(const void* a, const void* b, void* out, int64_t n, hipStream_t st
     T* op = static_cast<T*>(out);
     constexpr bool kGelu = OP == OP_GELU || OP == OP_GELU_ERF;  // (half types: gelu_half)
     constexpr bool kHalfLong = sizeof(T) == 2 && (OP == OP_SILU || OP == OP_SWIGLU);
-    constexpr int64_t kSingles = OP == OP_GELU ? kFewElems << 3 : kHalfLong ? kFewElems << 1 : kFewElems;
-    if (n <= kSingles && (sizeof(T) == 2 || kGelu || n >= kFewF32LightMin))
+    constexpr bool kLong = kHalfLong || OP == OP_GELU;
+    // (At addresses without 16-byte alignment runs pay off later: f32 GELU 0.5 M 3.3 µs in runs, 2.9 one by one, 1 M level.)
+    const bool at16 = aligned(ap, 16) && aligned(op, 16) && (OP != OP_SWIGLU || aligned(bp, 16));
+    const int64_t singles = kLong && !at16 ? kFewElems * 5 : kHalfLong ? kFewElems << 1 : kFewElems;
+    if (n <= singles && (sizeof(T) == 2 || kGelu || n >= kFewF32LightMin))
         return launch(ew_scalar<T, OP, BC>, grid_for(n, kThreads, 8192), kThreads, stream, ap, bp, op, n);
     const int64_t streams = (BC != B_SCALAR_A) + (binary_op<OP>() && BC != B_SCALAR_B) + 1;
     const int policy = policy_for(n * (int64_t)sizeof(T) * streams);

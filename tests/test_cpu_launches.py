@@ -146,3 +146,12 @@ def test_kv_slide_at_the_most_rows_a_launch_takes(launches):
     for seq in range((1 << 32) - 300, (1 << 32) - 256, 3):
         (st, ls), = launches(("sph_kv_cache_update", A, F16, B, F16, 1, seq, 8, seq + 1, 2, "host int64", None))
         assert st == 0 and ls, (seq, st)
+
+
+# One element a thread: f32 GELU to 2^18 elements, to 5 x 2^18 at addresses without 16-byte alignment.
+@pytest.mark.parametrize("off,n,kernel", [(0, 1 << 18, "scalar"), (0, (1 << 18) + 4, "runs"), (4, 5 << 18, "scalar"),
+                                          (4, (5 << 18) + 4, "runs")])
+def test_f32_gelu_kernel(launches, off, n, kernel):
+    for a, c in ((A + off, C), (A, C + off)):
+        (st, [(k, *_)]), = launches(("sph_gelu_tanh", a, c, F32, n, None))
+        assert st == 0 and k.startswith(f"ew_{kernel}<float,4,"), k
