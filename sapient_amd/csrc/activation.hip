@@ -62,9 +62,9 @@ constexpr int64_t kFewVecs = int64_t(1) << 20;
 
 // Smaller launches (decode steps, prefill chunks of small models) take one element per thread for
 // the ops whose per-element work is long: a thread's chain is then one element's, and all CUs have
-// work. Half-precision SiLU and SwiGLU up to 2^19 elements, then runs of four (8 bytes) up to 2^21,
-// then of eight: bf16 SwiGLU of 0.3 M elements 2.45 / 2.76 / 3.38 µs with one / four / eight, 1 M
-// 3.63 / 3.41 / 3.72, 3 M 6.88 / 6.01 / 5.73. GELU in f32 up to 2^18 (alone 0.3 M 2.41 µs against 3.07
+// work. Half-precision SiLU and SwiGLU up to 2^19 elements, then runs of eight: bf16 SwiGLU of 0.3 M
+// elements 2.45 / 3.38 µs with one / eight, 3 M 6.88 / 5.73 (runs of four, 2.76, 3.41 / 3.72 at 1 M and
+// 6.01, lose where the result is read next: f16 SwiGLU and an add 1 M 6.1 / 5.4, 2 M 8.3 / 6.8). GELU in f32 up to 2^18 (alone 0.3 M 2.41 µs against 3.07
 // with four and 1 M level, but between the bias that wrote its input and an add, the three 0.4 M
 // 7.9 / 7.1 µs, 1 M 12.0 / 9.0, 2 M 19.7 / 13.4). f32 SiLU and SwiGLU from 2048 elements up to 2^18
 // (0.3 M 2.35 / 2.5, 1 M 3.70 / 3.39; below 2048 level or 0.3 % slower); adds and products never
@@ -195,7 +195,7 @@ inline int policy_for(int64_t bytes) {
     return bytes >= kCachedBytes ? P_NT : bytes >= (int64_t(1) << 24) ? P_NT_STORES : P_CACHED;
 }
 
-// `n` elements in runs of E (16 bytes of T, or 8), U runs in flight per thread, at any element
+// `n` elements in runs of E (16 bytes of T), U runs in flight per thread, at any element
 // alignment; the thread whose run crosses the end takes its elements one by one, so odd sizes
 // and odd addresses are one launch too (512 x 4864 + 3 f32 8.4 -> 6.4 µs, 3000 x 5001 f16 at an odd
 // address, element by element before, 28.5 -> 18.0). B_SCALAR_B / B_SCALAR_A read element 0 of the
@@ -203,8 +203,9 @@ inline int policy_for(int64_t bytes) {
 // written, by the same thread. U = 1: the grid covers all runs, fewer than 2^31. (Issuing the
 // first loads before the exp table is staged costs 0.3 µs at 512 x 4864 f32 and 1.5 at bf16
 // 333 x 14336.) TAIL: n is no multiple of E (the tail's code alone costs a small launch 0.2 µs).
-template <typename T, int OP, int BC, int E, int U, int POLICY, bool TAIL>
+template <typename T, int OP, int BC, int U, int POLICY, bool TAIL>
 __global__ __launch_bounds__(kThreads) void ew_runs(const T* a, const T* b, T* out, int64_t n) {
+    constexpr int E = vec16<T>::n;
     constexpr bool NTL = POLICY == P_NT, NTS = POLICY != P_CACHED;
     using Index = std::conditional_t<U == 1, int32_t, int64_t>;
     __shared__ uint64_t exp_tab[needs_exp_table<OP, T>() ? 32 : 1];
@@ -279,30 +280,27 @@ int launch_ew(const void* a, const void* b, void* out, int64_t n, hipStream_t st
     constexpr bool kGelu = OP == OP_GELU || OP == OP_GELU_ERF;  // (half types: gelu_half)
     constexpr bool kHalfLong = sizeof(T) == 2 && (OP == OP_SILU || OP == OP_SWIGLU);
     constexpr bool kLong = kHalfLong || OP == OP_GELU;
-    // (At addresses without 16-byte alignment runs pay off later: f32 GELU 0.5 M 3.3 µs in runs, 2.9 one by one, 1 M level.)
+    // (At addresses without 16-byte alignment runs pay off later: f32 GELU 0.5 M 3.3 µs in runs, 2.9 one by one, 1 M level;
+    // f16 SwiGLU 0.8 M 3.8 / 3.4, 1.3 M 4.4 / 4.1, 1.6 M level.)
     const bool at16 = aligned(ap, 16) && aligned(op, 16) && (OP != OP_SWIGLU || aligned(bp, 16));
     const int64_t singles = kLong && !at16 ? kFewElems * 5 : kHalfLong ? kFewElems << 1 : kFewElems;
     if (n <= singles && (sizeof(T) == 2 || kGelu || n >= kFewF32LightMin))
         return launch(ew_scalar<T, OP, BC>, grid_for(n, kThreads, 8192), kThreads, stream, ap, bp, op, n);
     const int64_t streams = (BC != B_SCALAR_A) + (binary_op<OP>() && BC != B_SCALAR_B) + 1;
     const int policy = policy_for(n * (int64_t)sizeof(T) * streams);
-    auto go = [&](auto e, auto u, auto p) {
-        constexpr int EE = decltype(e)::value, U = decltype(u)::value;
-        const unsigned grid = grid_for((n + EE - 1) / EE, (int64_t)kThreads * U, kMaxGrid);
-        return n % EE == 0
-                   ? launch(ew_runs<T, OP, BC, EE, U, decltype(p)::value, false>, grid, kThreads, stream, ap, bp, op, n)
-                   : launch(ew_runs<T, OP, BC, EE, U, decltype(p)::value, true>, grid, kThreads, stream, ap, bp, op, n);
+    auto go = [&](auto u, auto p) {
+        constexpr int U = decltype(u)::value;
+        const unsigned grid = grid_for((n + E - 1) / E, (int64_t)kThreads * U, kMaxGrid);
+        return n % E == 0 ? launch(ew_runs<T, OP, BC, U, decltype(p)::value, false>, grid, kThreads, stream, ap, bp, op, n)
+                          : launch(ew_runs<T, OP, BC, U, decltype(p)::value, true>, grid, kThreads, stream, ap, bp, op, n);
     };
-    const std::integral_constant<int, E> run;
     const std::integral_constant<int, 1> one;
     const std::integral_constant<int, kUnroll> two;
     const std::integral_constant<int, P_CACHED> cached;
     const std::integral_constant<int, P_NT_STORES> nt_stores;
     const std::integral_constant<int, P_NT> nt;
-    if constexpr (kHalfLong)
-        if (n <= kFewElems << 3) return go(std::integral_constant<int, 4>{}, one, cached);
-    if ((n + E - 1) / E <= kFewVecs) return policy == P_CACHED ? go(run, one, cached) : go(run, one, nt_stores);
-    return policy == P_NT ? go(run, two, nt) : go(run, two, nt_stores);
+    if ((n + E - 1) / E <= kFewVecs) return policy == P_CACHED ? go(one, cached) : go(one, nt_stores);
+    return policy == P_NT ? go(two, nt) : go(two, nt_stores);
 }
 
 template <int OP>

@@ -155,3 +155,14 @@ def test_f32_gelu_kernel(launches, off, n, kernel):
     for a, c in ((A + off, C), (A, C + off)):
         (st, [(k, *_)]), = launches(("sph_gelu_tanh", a, c, F32, n, None))
         assert st == 0 and k.startswith(f"ew_{kernel}<float,4,"), k
+
+
+# Half SiLU and SwiGLU: one element a thread to 2^19 elements (5 x 2^18 unaligned), else whole runs.
+@pytest.mark.parametrize("off,n,kernel", [(0, 1 << 19, "scalar"), (0, (1 << 19) + 8, "runs"), (2, 5 << 18, "scalar"),
+                                          (8, (5 << 18) + 8, "runs")])
+def test_half_silu_kernel(launches, off, n, kernel):
+    calls = [("sph_silu", A + off, C, F16, n, None), ("sph_swiglu", A, B + off, C, F16, n, None)]
+    for call in calls:
+        (st, [(k, x, _, b)]), = launches(call)
+        assert st == 0 and k.startswith(f"ew_{kernel}<"), k
+        assert kernel == "scalar" or x * b >= n // 8 > x * b - b, (k, x, b)
