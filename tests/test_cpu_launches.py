@@ -166,3 +166,13 @@ def test_half_silu_kernel(launches, off, n, kernel):
         (st, [(k, x, _, b)]), = launches(call)
         assert st == 0 and k.startswith(f"ew_{kernel}<"), k
         assert kernel == "scalar" or x * b >= n // 8 > x * b - b, (k, x, b)
+
+
+# Where one run a thread covers a launch: cached below 16 MB of traffic (policy 0), non-temporal from there on (2).
+@pytest.mark.parametrize("n,policy", [((1 << 20) + 4, 0), (1 << 21, 2), (1 << 22, 2)])
+def test_element_wise_cache_policy(launches, n, policy):
+    for call in (("sph_add", A, n, B, n, C, F32, None), ("sph_mul", A, n, B, 1, C, F32, None),
+                 ("sph_swiglu", A, B, C, F32, n, None)):
+        (st, [(k, *_)]), = launches(call)
+        u, p = map(int, k.split(",")[3:5])
+        assert st == 0 and (u != 1 or p == policy), k
