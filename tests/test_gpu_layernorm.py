@@ -141,7 +141,7 @@ def test_layer_norm_kat(dev):
     assert np.abs(out - np.array([[-1, 1], [-1, 1]])).max() < 1e-4
 
 
-def test_layer_norm_unaligned_views_take_generic_path(dev, orc):
+def test_layer_norm_unaligned_views(dev, orc):
     base = _gen((4 * 768 + 1,), 91, dev, 1.0, 2.0)
     x = base[1:].view(4, 768)
     out = torch.empty(4 * 768 + 1, device=dev)[1:].view(4, 768)

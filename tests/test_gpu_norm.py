@@ -79,7 +79,7 @@ def test_rms_norm_shapes(dev, orc, dtype, rows, dim, wmode, outmode):
                                       (600, 1024), (3, 100)])
 def test_add_rms_norm_shapes(dev, orc, dtype, rows, dim):
     """Widths that take each launch shape: the row-looping one (up to 4096 f32 / 8192 half
-    elements), one block per row, twice the values per lane past 16 waves, and the generic kernel."""
+    elements), one block per row, twice the values per lane past 16 waves, and (rows of 100 halves) the generic kernel."""
     print(f"case add_rms_norm {dtype} {rows}x{dim}", flush=True)
     x = _gen((rows, dim), 11 + dim, dev, dtype=dtype)
     r = _gen((rows, dim), 13 + dim, dev, dtype=dtype)
@@ -126,7 +126,7 @@ def test_add_rms_norm_to_equals_in_place(dev, orc, dtype, rows, dim):
 
 
 def test_add_rms_norm_to_unaligned_and_half_outputs(dev, orc):
-    """The generic kernel (a 4-byte offset view) and an f16 output with an f16 weight, out of place."""
+    """The ragged kernel (a 4-byte offset view) and an f16 output with an f16 weight, out of place."""
     base = _gen((4 * 896 + 1,), 61, dev)
     x = base[1:].view(4, 896)
     r = _gen((4, 896), 62, dev)
@@ -180,8 +180,8 @@ def test_rms_norm_kat(dev):
     assert abs(out[0, 0].item() - e0) < 1e-5 and abs(out[0, 1].item() - e1) < 1e-5
 
 
-def test_rms_norm_unaligned_views_take_generic_path(dev, orc):
-    """Pointers that are not 16-byte aligned must still be correct (generic kernel)."""
+def test_rms_norm_unaligned_views(dev, orc):
+    """Pointers that are not 16-byte aligned must still be correct (rows in runs at element alignment)."""
     base = _gen((4 * 896 + 1,), 41, dev)
     x = base[1:].view(4, 896)  # 4-byte offset
     out = torch.empty(4 * 896 + 1, device=dev)[1:].view(4, 896)

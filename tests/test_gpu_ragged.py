@@ -77,8 +77,10 @@ def test_ragged_norms(dev, orc, dtype, rows, dim, off):
 
 
 # Element-wise launches around every bound of their dispatch (2^18 .. 2^21 elements, 2^20 vectors, 16 and 128 MB of
-# traffic), a few elements past each (short last runs) and at odd addresses, against the same op over pieces of at
-# most 2^18 elements at aligned addresses: the one-element kernel, which the other tests check against the oracle.
+# traffic), a few elements past each (short last runs) and at odd addresses. Every element against the same op over
+# pieces of at most 2^18 elements at aligned addresses, which take the one-element kernel (f32 SiLU and SwiGLU pieces
+# below 2048 elements, adds and products in f32 as well: runs); the first and last elements, where a launch's short runs
+# are, against the oracle; adds and products against torch throughout.
 def _pieces(fn, *xs):
     step = 1 << 18
     n = max(x.numel() for x in xs)
@@ -90,7 +92,7 @@ def _pieces(fn, *xs):
 @pytest.mark.parametrize("n", [1, 2049, (1 << 18) + 1, (1 << 19) - 3, (1 << 19) + 8, (1 << 20) + 5, (1 << 21) + 2,
                                (1 << 22) + 4, (1 << 22) + 7, (1 << 23) + 1, 23_000_000])
 @pytest.mark.parametrize("off", [0, 1])
-def test_elementwise_launch_bounds(dev, dtype, n, off):
+def test_elementwise_launch_bounds(dev, orc, dtype, n, off):
     print(f"case elementwise {dtype} n {n} offset {off}", flush=True)
     x, u = _gen((n,), 11, dev, dtype, off, 2.0), _gen((n,), 12, dev, dtype, off, 2.0)
     one = _gen((1,), 13, dev, dtype)
@@ -102,6 +104,16 @@ def test_elementwise_launch_bounds(dev, dtype, n, off):
     if n > 1:
         same(ops.add(x, one), _pieces(ops.add, x, one), "add scalar")
         same(ops.mul(one, x), _pieces(ops.mul, one, x), "scalar mul")
+    for fn, tf in ((ops.add, torch.add), (ops.mul, torch.mul)):  # in f32, rounded once
+        same(fn(x, u), tf(x.float(), u.float()).to(dtype), "against torch")
+        same(fn(x, one), tf(x.float(), one.float()).to(dtype), "by a scalar, against torch")
+    ends = torch.cat([x[:1100], x[-1100:]]), torch.cat([u[:1100], u[-1100:]])
+    x32, u32 = (widen(t, orc) for t in ends)
+    pick = lambda y: torch.cat([y[:1100], y[-1100:]])
+    _same(pick(ops.silu(x)), orc.silu(x32), dtype, orc, "silu ends")
+    _same(pick(ops.swiglu(x, u)), orc.swiglu(x32, u32), dtype, orc, "swiglu ends")
+    _same(pick(ops.gelu_tanh(x)), orc.gelu(x32), dtype, orc, "gelu_tanh ends")
+    _same(pick(ops.gelu_erf(x)), orc.gelu_erf(x32), dtype, orc, "gelu_erf ends")
     want = _pieces(ops.swiglu, x, u)
     assert ops.swiglu(x, u, out=x) is x  # in place
     same(x, want, "swiglu in place")
