@@ -581,4 +581,11 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_torch_ops", nullptr, -1, kMethod
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__torch_ops() { return PyModule_Create(&kModule); }
+PyMODINIT_FUNC PyInit__torch_ops() {
+    PyObject* m = PyModule_Create(&kModule);
+    // What it was built for: torch's C++ ABI changes with its version.
+    if (m && (PyModule_AddStringConstant(m, "torch_version", SPH_TORCH_VERSION) < 0 ||
+              PyModule_AddIntConstant(m, "abi_version", SPH_ABI_VERSION) < 0))
+        Py_CLEAR(m);
+    return m;
+}

@@ -5,18 +5,22 @@ host layer (``host/*.cpp``) is compiled by hipcc (in parallel) into
 ``sapient_amd/_build/`` and linked into one shared library that exports the C
 ABI declared in ``include/sapient_hip.h`` and the C++ API of
 ``include/sapient_hip_backend.hpp``. The native half of :mod:`sapient_amd.ops`
-(``binding/torch_ops.cpp``, against torch's headers) is compiled by g++ into
-``sapient_amd/_torch_ops.so``, which links that library.
+(``binding/torch_ops.cpp``, against the headers of Python and of the installed
+torch) is compiled into ``sapient_amd/_torch_ops.so``, which links that library;
+where torch or Python's headers are missing it is left out, with a note: the
+library needs hipcc alone.
 
 Usage: ``python -m sapient_amd.build`` (or ``__graft_entry__.build()``).
 """
 from __future__ import annotations
 
 import concurrent.futures as cf
+import importlib.util
 import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
@@ -73,23 +77,30 @@ def _compile(src: Path) -> Path:
     return obj
 
 
-def _build_binding() -> None:
-    """The torch binding: host code only, in torch's own C++ ABI, found beside the library at run time."""
-    import sysconfig
-
+def _build_binding() -> str:
+    """The torch binding: host code only, in torch's own C++ ABI, found beside the library at run time.
+    Returns why it was left out, or "". It records the torch and the ABI it was built for (ops.py checks both)."""
+    include = Path(sysconfig.get_paths()["include"])
+    missing = ("torch" if importlib.util.find_spec("torch") is None else
+               "Python.h" if not (include / "Python.h").exists() else "")
+    if missing:
+        BINDING.unlink(missing_ok=True)  # one from an earlier build would be for another library
+        return f"{missing} not found"
     import torch
     t = Path(torch.__file__).parent
     tmp = BINDING.with_suffix(".so.tmp")
-    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
-           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}", f"-I{ROOT / 'include'}",
+    cmd = [shutil.which("g++") or hipcc(), "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1",
+           "-DUSE_ROCM=1", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+           f'-DSPH_TORCH_VERSION="{torch.__version__}"', f"-I{ROOT / 'include'}",
            "-isystem", str(t / "include"), "-isystem", str(t / "include" / "torch" / "csrc" / "api" / "include"),
-           "-isystem", "/opt/rocm/include", "-isystem", sysconfig.get_paths()["include"],
+           "-isystem", "/opt/rocm/include", "-isystem", str(include),
            str(PKG / "binding" / "torch_ops.cpp"), "-o", str(tmp), f"-L{PKG}", f"-l:{LIB.name}", f"-L{t / 'lib'}",
            "-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip", "-Wl,-rpath,$ORIGIN"]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
-        raise RuntimeError(f"g++ failed for torch_ops.cpp:\n{res.stderr}")
+        raise RuntimeError(f"{cmd[0]} failed for torch_ops.cpp:\n{res.stderr}")
     os.replace(tmp, BINDING)
+    return ""
 
 
 def build(verbose: bool = True) -> Path:
@@ -106,9 +117,11 @@ def build(verbose: bool = True) -> Path:
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stderr}")
     os.replace(tmp, LIB)
-    _build_binding()
+    left_out = _build_binding()
     if verbose:
         print(f"built {LIB.relative_to(ROOT)} from {len(srcs)} sources")
+        if left_out:
+            print(f"left out {BINDING.relative_to(ROOT)}, the calls on torch tensors: {left_out}")
     return LIB
 
 

@@ -36,6 +36,10 @@ class _Unloaded:
             from . import _torch_ops
         except ImportError as e:
             raise RuntimeError(f"_torch_ops.so is not built or does not load ({e}); run `python -m sapient_amd.build`") from e
+        built = (_torch_ops.torch_version, _torch_ops.abi_version)
+        if built != (str(torch.__version__), lib().sph_abi_version()):
+            raise RuntimeError(f"_torch_ops.so is built for torch {built[0]} and ABI {built[1]}, not torch {torch.__version__} "
+                               f"and ABI {lib().sph_abi_version()}; run `python -m sapient_amd.build`")
         _torch_ops.set_check(check)
         _native = _torch_ops
         return getattr(_torch_ops, name)

@@ -29,3 +29,23 @@ def test_refuses_host_tensors_and_other_objects(name):
         CALLS[name](X)
     with pytest.raises(TypeError, match="must be a torch.Tensor"):
         CALLS[name](object())
+
+
+def test_library_builds_without_torch(monkeypatch, tmp_path):
+    """The C library needs hipcc alone: without torch the binding is left out, and none from an earlier build stays."""
+    from sapient_amd import build
+    stale = tmp_path / "_torch_ops.so"
+    stale.write_bytes(b"an earlier build")
+    monkeypatch.setattr(build, "BINDING", stale)
+    monkeypatch.setattr(build.importlib.util, "find_spec", lambda name: None)
+    assert build._build_binding() == "torch not found" and not stale.exists()
+
+
+@pytest.mark.parametrize("what", ["torch", "abi"])
+def test_refuses_a_binding_built_for_another(monkeypatch, what):
+    if what == "torch":
+        monkeypatch.setattr(torch, "__version__", "0.0.1")
+    else:
+        monkeypatch.setattr(ops, "lib", lambda: type("L", (), {"sph_abi_version": staticmethod(lambda: 99)}))
+    with pytest.raises(RuntimeError, match="is built for torch .* run `python -m sapient_amd.build`"):
+        ops._Unloaded().silu
