@@ -124,6 +124,11 @@ int32_t* flag(PyObject* o, const char* name) {
     return static_cast<int32_t*>(t.data_ptr());
 }
 
+struct NoGil {
+    PyThreadState* state = PyEval_SaveThread();
+    ~NoGil() { PyEval_RestoreThread(state); }
+};
+
 // The caller's output, after checking that it holds exactly what the kernel writes, or a fresh one.
 struct Out {
     PyObject* given;
@@ -131,6 +136,8 @@ struct Out {
     Out(PyObject* o, at::IntArrayRef shape, ScalarType dtype, at::Device device, const char* name = "out")
         : given(o == Py_None ? nullptr : o) {
         if (!given) {
+            // Without the GIL, as torch's own calls: the allocator may wait for its lock, or for the device.
+            const NoGil release;
             t = at::empty(shape, at::TensorOptions().dtype(dtype).device(device));
             return;
         }

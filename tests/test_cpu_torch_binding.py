@@ -1,5 +1,9 @@
 """The native op calls (binding/torch_ops.cpp) without a GPU: every function of ops.py reaches its argument
 checks with the arguments it documents, and refuses what is not a contiguous device tensor."""
+import subprocess
+import sys
+from pathlib import Path
+
 import pytest
 import torch
 
@@ -49,3 +53,32 @@ def test_refuses_a_binding_built_for_another(monkeypatch, what):
         monkeypatch.setattr(ops, "lib", lambda: type("L", (), {"sph_abi_version": staticmethod(lambda: 99)}))
     with pytest.raises(RuntimeError, match="is built for torch .* run `python -m sapient_amd.build`"):
         ops._Unloaded().silu
+
+
+CHILD = """
+import ctypes, sys
+import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
+with FakeTensorMode():
+    x = torch.empty(8, device="cuda")  # passes for a device tensor; there is no memory behind it
+seen = ctypes.PyDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+import sapient_amd.ops as ops
+try:
+    ops.silu(x)
+except RuntimeError as e:
+    print(e, seen.empty_calls(), seen.empty_held())
+"""
+
+
+def test_outputs_are_allocated_without_the_gil():
+    """As by torch's own calls: other Python threads run on while the allocator waits for its lock or the device."""
+    root = Path(__file__).resolve().parents[1]
+    so = root / "tests" / "native" / "_build" / "empty_recorder.so"
+    if not so.exists():
+        import importlib.util
+        spec = importlib.util.spec_from_file_location("native_build", so.parents[1] / "build.py")
+        mod = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(mod)
+        mod.build()
+    res = subprocess.run([sys.executable, "-c", CHILD, str(so)], capture_output=True, text=True, cwd=root, timeout=120)
+    assert res.stdout.split() == ["recorded", "1", "0"], res.stdout + res.stderr
