@@ -305,9 +305,12 @@ int sph_kv_append(const void* src, int src_dtype, void* cache, int cache_dtype, 
  * cur_len > max_seq SPH_EINVAL; nothing is written then, nor when the append
  * itself would be rejected (its checks run before the shift). Types,
  * conversion and the Q8_0 layout are sph_kv_append's. The shift runs in place,
- * in two launches per 65535 heads, and moves each kept row once where it is
- * small against the rows a block holds (at least 31 f16 rows of 128), else
- * twice; the append rides in the second launch where the cache's rows split
+ * in two launches per 65535 heads. Each kept row moves twice, or, where the
+ * shift is small against the rows a block holds (at most 31 f16 rows of 128) and
+ * the valid rows are of 5 MB or more, once except that `shift` rows of every
+ * window (a block's rows) move twice. One launch does where a block holds a whole
+ * head; a head of more than 4096 windows, 262144 f16 rows of 128, moves its rows
+ * twice. The append rides in the last launch where the cache's rows split
  * into aligned 16-byte units, else it is a launch of its own. The rows moved
  * by the shift are copied bit for bit, and the shift's rows past
  * cur_len - shift hold intermediate values until the append overwrites them.

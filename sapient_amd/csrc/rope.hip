@@ -60,17 +60,10 @@ struct TableArgs {
     int32_t* bad;
 };
 
+// The large-argument reduction indexes the 4/pi table per lane; staged in LDS (by each kernel, before its angles)
+// the lookups stay off the vector-memory queue the row stream keeps full (measured: ~1.5 µs of 58 at the
+// Llama-3-8B shape).
 __constant__ InvPio4Table kInvPio4 = inv_pio4_table();
-
-// The large-argument reduction indexes the 4/pi table per lane; staged in LDS
-// the lookups stay off the vector-memory queue the row stream keeps full
-// (measured: ~1.5 µs of 58 at the Llama-3-8B shape). Every thread of the block
-// must call this before any returns.
-__device__ __forceinline__ const uint32_t* stage_inv_pio4(uint32_t (&tab)[24]) {
-    if (threadIdx.x < 24) tab[threadIdx.x] = kInvPio4.w[threadIdx.x];
-    __syncthreads();
-    return tab;
-}
 
 // L consecutive elements of one row held as they sit in memory (32-bit words,
 // or single elements when the run is narrower than a word or ELEM asks for
