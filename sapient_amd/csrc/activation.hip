@@ -40,6 +40,7 @@
 //    the ones of the tanh form.
 //  - Bias add: a block owns a tile of up to 256 16-byte column runs over
 //    two rows; each thread loads its bias vector once and adds it to both.
+//    Narrow or small rows that no aligned vector fits go element by element.
 #include <mutex>
 #include <type_traits>
 
@@ -64,12 +65,12 @@ constexpr int64_t kFewVecs = int64_t(1) << 20;
 // the ops whose per-element work is long: a thread's chain is then one element's, and all CUs have
 // work. Half-precision SiLU and SwiGLU up to 2^19 elements, then runs of eight: bf16 SwiGLU of 0.3 M
 // elements 2.45 / 3.38 µs with one / eight, 3 M 6.88 / 5.73 (runs of four, 2.76, 3.41 / 3.72 at 1 M and
-// 6.01, lose where the result is read next: f16 SwiGLU and an add 1 M 6.1 / 5.4, 2 M 8.3 / 6.8). GELU in f32 up to 2^18 (alone 0.3 M 2.41 µs against 3.07
-// with four and 1 M level, but between the bias that wrote its input and an add, the three 0.4 M
-// 7.9 / 7.1 µs, 1 M 12.0 / 9.0, 2 M 19.7 / 13.4). f32 SiLU and SwiGLU from 2048 elements up to 2^18
-// (0.3 M 2.35 / 2.5, 1 M 3.70 / 3.39; below 2048 level or 0.3 % slower); adds and products never
-// gain. Half-precision GELU reads its table from cache up to kFewElems instead of staging it per
-// block (1 x 10240 f16 2.90 -> 1.79 µs). Results are the same bits either way.
+// 6.01, lose where the result is read next: f16 SwiGLU and an add 1 M 6.1 / 5.4, 2 M 8.3 / 6.8). GELU
+// in f32 up to 2^18 (alone 0.3 M 2.41 µs against 3.07 with four and 1 M level, but between the bias that
+// wrote its input and an add, the three 0.4 M 7.9 / 7.1 µs, 1 M 12.0 / 9.0, 2 M 19.7 / 13.9). f32 SiLU
+// and SwiGLU from 2048 elements up to 2^18 (0.3 M 2.35 / 2.5, 1 M 3.70 / 3.39; below 2048 level or 0.3 %
+// slower); adds and products never gain. Half-precision GELU reads its table from cache up to kFewElems
+// instead of staging it per block (1 x 10240 f16 2.90 -> 1.79 µs). Results are the same bits either way.
 constexpr int64_t kFewElems = int64_t(1) << 18;
 constexpr int64_t kFewF32LightMin = 2048;
 
@@ -196,7 +197,7 @@ inline int policy_for(int64_t bytes) {
 }
 
 // `n` elements in runs of E (16 bytes of T), U runs in flight per thread, at any element
-// alignment; the thread whose run crosses the end takes its elements one by one, so odd sizes
+// alignment; the thread whose run crosses the end takes its elements in pieces, so odd sizes
 // and odd addresses are one launch too (512 x 4864 + 3 f32 8.4 -> 6.4 µs, 3000 x 5001 f16 at an odd
 // address, element by element before, 28.5 -> 18.0). B_SCALAR_B / B_SCALAR_A read element 0 of the
 // broadcast operand. `out` may alias a full-length input: each element is read before it is
@@ -299,11 +300,15 @@ int launch_ew(const void* a, const void* b, void* out, int64_t n, hipStream_t st
     const std::integral_constant<int, P_CACHED> cached;
     const std::integral_constant<int, P_NT_STORES> nt_stores;
     const std::integral_constant<int, P_NT> nt;
-    // One run per thread: past 16 MB both ways non-temporal. Alone, cached loads are as fast or up to 7 % faster (above),
-    // but reading what a kernel has just written they are slower: an add, then a product with a scalar, f32 3 M 12.1
-    // against 9.4 µs, f16 8 M 15.5 / 11.9; SwiGLU, then an add, f32 3 M 15.3 / 12.4, f16 6 M 15.8 / 13.4; bias, GELU, add
-    // f32 4 M 24.0 / 21.5.
-    if ((n + E - 1) / E <= kFewVecs) return policy == P_CACHED ? go(one, cached) : go(one, nt);
+    // One run per thread: adds and products past 16 MB both ways non-temporal. They read what a kernel has just written,
+    // and cached loads of that are slower: an add, then a product with a scalar, f32 3 M 12.1 against 9.1 µs, f16 8 M
+    // 15.5 / 11.7; SwiGLU, then an add, f32 3 M 15.4 / 13.4. The activations keep cached loads: on inputs written longer
+    // ago SwiGLU f32 512 x 4864 takes 6.8 µs against 7.6 non-temporal, bf16 333 x 14336 6.9 / 8.0.
+    if ((n + E - 1) / E <= kFewVecs) {
+        if (policy == P_CACHED) return go(one, cached);
+        if constexpr (OP == OP_ADD || OP == OP_MUL) return go(one, nt);
+        else return go(one, nt_stores);
+    }
     return policy == P_NT ? go(two, nt) : go(two, nt_stores);
 }
 
@@ -392,7 +397,7 @@ __device__ __forceinline__ uint32_t gelu_lookup(const uint16_t* tab, uint32_t h)
 
 // Blocks of THREADS that each stage the band table in LDS once and then stream
 // 16-byte runs, grid-stride, U per thread per trip, at any element alignment (the
-// thread whose run crosses the end takes its elements one by one), past the
+// thread whose run crosses the end takes its elements in pieces), past the
 // caches at every size: erf-GELU f16 after the bias that wrote its input, 1500 x
 // 5120, 7.5 µs against 8.8 with cached loads and 3000 x 5120 14.2 against 17.2.
 //  - Up to one trip of 1024 threads x 4 runs on every CU (8 M elements): one block

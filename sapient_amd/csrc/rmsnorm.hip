@@ -244,10 +244,10 @@ __global__ __launch_bounds__(W >= 4 ? 64 * W : 256) void rms_rows_vec(const TX* 
 // Rows whose width no 16-byte vector divides, or whose pointers are only element-aligned: the row
 // is split and held in registers as in rms_rows_vec (one read of every input), each lane moving
 // 16-byte runs at whatever alignment its row has; the lane whose run crosses the row's end moves
-// its last elements one by one. HBM-bound; the straddled cache lines cost about a third over the
-// aligned kernel. Against rms_rows_generic (three passes of element accesses) on MI355X: add +
-// RMSNorm f16 4099 x 2565 29.1 -> 20.7 µs, f32 53.4 -> 31.2, bf16 16384 x 4095 222 -> 145; RMSNorm
-// bf16 16384 x 4095 143 -> 74; LayerNorm 176 -> 80. Shifting every lane's runs to 16- or 128-byte
+// its last elements in pieces (f32: one by one). HBM-bound; the straddled cache lines cost about a
+// third over the aligned kernel. Against rms_rows_generic (three passes of element accesses) on MI355X:
+// add + RMSNorm f16 4099 x 2565 29.1 -> 17.9 µs, f32 53.4 -> 31.2, f16 20000 x 4097 275 -> 138; RMSNorm
+// 176 -> 79; LayerNorm 213 -> 92. Shifting every lane's runs to 16- or 128-byte
 // boundaries of the row (all full runs aligned) was slower in every case (RMSNorm 74 -> 82-83):
 // both ends of a row then move element by element.
 // weight and bias are f32 (wb_f32) or TX.
@@ -461,8 +461,8 @@ int launch_ragged(const TX* xp, TX* rp, TX* sp, const void* wp, const void* bp, 
 // Runs per lane of a ragged launch: one where the launch is small (up to kFewValues; f16 300 x 1001
 // 4.1 µs against 4.8 with two) or fuses an f32 add (4096 x 4096 at an odd offset 45.8 against 50.5),
 // else two (RMSNorm bf16 16384 x 4095 74 against 88, LayerNorm 80 against 97). Cached accesses
-// up to kCachedBytes: f16 add 4099 x 2565 (84 MB) 20.7 against 24.2 non-temporal, at 134 MB both
-// alike, bf16 16384 x 4095 (537 MB) 152 against 145.
+// up to kCachedBytes: f16 add 4099 x 2565 (84 MB, row ends element by element) 20.7 against 24.2
+// non-temporal, at 134 MB both alike, bf16 16384 x 4095 (537 MB) 152 against 145.
 template <typename TX, typename TO, int KIND>
 int launch_ragged_any(const TX* xp, TX* rp, TX* sp, const void* wp, const void* bp, bool wb_f32, TO* op, int64_t nr,
                       int64_t dim, float eps, bool few, hipStream_t stream) {

@@ -168,11 +168,13 @@ def test_half_silu_kernel(launches, off, n, kernel):
         assert kernel == "scalar" or x * b >= n // 8 > x * b - b, (k, x, b)
 
 
-# Where one run a thread covers a launch: cached below 16 MB of traffic (policy 0), non-temporal from there on (2).
-@pytest.mark.parametrize("n,policy", [((1 << 20) + 4, 0), (1 << 21, 2), (1 << 22, 2)])
-def test_element_wise_cache_policy(launches, n, policy):
-    for call in (("sph_add", A, n, B, n, C, F32, None), ("sph_mul", A, n, B, 1, C, F32, None),
-                 ("sph_swiglu", A, B, C, F32, n, None)):
+# Where one run a thread covers a launch: cached below 16 MB of traffic (policy 0), from there on non-temporal stores
+# (1), for adds and products loads as well (2).
+@pytest.mark.parametrize("n", [(1 << 20) + 4, 1 << 21, 1 << 22])
+def test_element_wise_cache_policy(launches, n):
+    large = n >= 1 << 21
+    for call, want in ((("sph_add", A, n, B, n, C, F32, None), 2 * large), (("sph_mul", A, n, B, 1, C, F32, None), 2 * large),
+                       (("sph_swiglu", A, B, C, F32, n, None), large), (("sph_gelu_erf", A, C, F32, n, None), large)):
         (st, [(k, *_)]), = launches(call)
         u, p = map(int, k.split(",")[3:5])
-        assert st == 0 and (u != 1 or p == policy), k
+        assert st == 0 and (u, p) == (1, want), k
