@@ -75,13 +75,7 @@ __device__ __forceinline__ float row_sum(float v, float (*partial)[WPB], int slo
 template <typename T, int E>
 __device__ __forceinline__ void unpack16(const u32x4& q, float (&v)[E]) {
     const uint32_t raw[4] = {q.x, q.y, q.z, q.w};
-    if constexpr (sizeof(T) == 4) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = __uint_as_float(raw[i]);
-    } else {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = widen(T{(uint16_t)(raw[i / 2] >> (16 * (i & 1)))});
-    }
+    words_to_f32<T, E>(raw, v);
 }
 
 // W waves per row, VPT 16-byte vectors per lane, RPB rows per block.
