@@ -136,7 +136,8 @@ struct Out {
     Out(PyObject* o, at::IntArrayRef shape, ScalarType dtype, at::Device device, const char* name = "out")
         : given(o == Py_None ? nullptr : o) {
         if (!given) {
-            // Without the GIL, as torch's own calls: the allocator may wait for its lock, or for the device.
+            // Without the GIL, as torch's own calls: the allocator may wait for its lock, or for the device. (It
+            // costs a decode step's five calls 0.35 µs, 22.5 -> 22.85.)
             const NoGil release;
             t = at::empty(shape, at::TensorOptions().dtype(dtype).device(device));
             return;
